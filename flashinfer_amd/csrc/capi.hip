@@ -302,11 +302,10 @@ Variants pick_variants(int64_t T) {
     // 419.4 against 422.6, T=1024 364.6 against 370.5 and 221.0 against
     // 224.1 at two shard offsets).
     else if (T <= 1536) v = {15, 21};
-    // GEMM1 LDS tile as one software pipeline (barriers inside the MFMA
-    // stream, weight fragments held in registers): bitwise equal to variant
-    // 18 and faster at every T (GEMM1 per launch, one process: T=8192 401-420
-    // against 436-509 us, T=14000 skewed 2972 against 3151, T=3072 287
-    // against 308); level with the wide kernel at T=2048.
+    // GEMM1 LDS tile with two wave groups that take turns at the matrix cores:
+    // bitwise equal to variants 3 and 18 and faster at every T (GEMM1 per launch,
+    // one process: T=8192 428-440 against 482-486 us for variant 18, T=14000
+    // skewed 2,690-2,747 against 3,083-3,111, T=2048 177-181 against 214-223).
     else v = {19, 21};
     // From T = 640 to 1536 the GEMM1 kernel is chosen on the device from the
     // expert counts (G1_SELECT_EXTRA_TILES): the wide kernel streams an

@@ -394,56 +394,79 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm1_tile_t_kernel(
     }
 }
 
-// The same 256 x (128 + 128) tile as one software pipeline (variant 19).
+// The same 256 x (128 + 128) tile with its waves in two groups that take turns
+// at the matrix cores (variant 19).
 //
-// The 8 waves form 2 row groups x 4 column groups: wave (wm, wn) owns rows
-// 128wm .. 128wm+127 (8 row tiles of 16) and gate columns 32wn .. 32wn+31
-// (2 column tiles) plus the matching up columns, 32 MFMAs per k-block as in
-// variants 3 and 18. A wave keeps its four weight fragments of a k-block in
-// registers (32 VGPRs) and streams the 8 activation fragments from LDS. The
-// two barriers of a k-block sit inside the MFMA stream, so no wave waits on
-// LDS or on a barrier with an empty matrix core queue:
-//   * barrier X, after row tile 0: every wave has its weight fragments of
-//     k-block kb in registers (read during k-block kb-1), so that stage's
-//     weight region is free and the copy of the weights of k-block kb+2 goes
-//     there: a weight copy has ~1.75 k-blocks to arrive;
-//   * barrier Y, before row tile 7: the copies of k-block kb+1 have landed
-//     (vmcnt leaves only the weights of kb+2 outstanding), and every wave has
-//     read its last activation fragment of kb, so the activation rows of
-//     k-block kb+2 are copied into this stage's activation region (one
-//     k-block to arrive). During row tile 7 each wave reads the next
-//     k-block's weight fragments into the same registers right after their
-//     last MFMA, its first activation fragment and its row scales.
-// Weights are the operand that comes from HBM (an expert's column tile is
-// read by its few row tiles, an activation row tile by all 16 column tiles).
-// MFMA operands are swapped as in variant 18 (weights are the A operand, so
-// a lane holds four output columns of one row and one scale factor per
-// tile), and each MFMA's four scale FMAs issue after the MFMA four later
-// (the next row tile's, same column tile); the last row tile's carry into
-// the next k-block.
-struct G1W {
+// Waves 0-3 (group 0: rows 0-127) and 4-7 (group 1: rows 128-255) share the
+// four SIMDs, one wave of each group per SIMD; wave wn of a group owns 32
+// gate columns and the matching 32 up columns. A k-block is four phases per
+// wave, a barrier after each, and group 1 runs one phase behind group 0:
+//   M0: read the weight fragments and row tiles 0-3 from LDS
+//   C0: their 16 MFMAs
+//   M1: read row tiles 4-7
+//   C1: their 16 MFMAs
+// so in every slot one wave of a SIMD multiplies from registers while the
+// other one reads LDS, issues copies and applies the last scale factors. What
+// bounded the one-group pipeline this replaces was LDS reads and barriers
+// with an empty matrix core queue (all waves read their fragments at the same
+// time): 2,657 cycles a k-block now against about 4,450 before, 2,048 of
+// them MFMA. The rest is power: with random data the clock falls to 1.6-1.8
+// GHz in this loop (2.1-2.2 in the same loop without its copies), so bytes
+// and operations saved count as much as cycles. GEMM1 alone, one process: T=14000 with every
+// token on 8 experts 3,010 -> 2,695 us, T=8192 458 -> 420 us (medians).
+//
+// Copies (two stages): the weights and row tiles 0-3 of k-block kb + 2 go out
+// in M1 of kb, after both groups have read theirs of kb (group 1 in the slot
+// before); row tiles 4-7 of kb + 1 go out in M0 of kb. Either has six slots
+// (1.5 k-blocks) to land. The copies that the next slot's readers need are
+// waited for by the wave that issued them (vmcnt of the NV copies issued
+// since) before the barrier that ends the slot: for group 0 that is the end
+// of C0 / C1, for group 1, one slot behind, the end of M0 / M1.
+//
+// A tile of at most 128 rows gives each group 64 of them (M, C; two phases a
+// k-block, a third of the activation copies) and uses the LDS for three
+// stages. An expert's last row tile is often one: at T=1000 (19 row tiles)
+// 144 -> 133 us.
+//
+// MFMA operands are swapped as in variant 18 (weights are the A operand, so a
+// lane holds four output columns of one row and one scale factor per tile),
+// and each MFMA's four scale FMAs issue LAG MFMAs later; the last ones of a
+// phase run in the M phase after it. Same products and order of sums as
+// variants 3 and 18, bitwise.
+struct G1P {
     static constexpr int NW = 8;
     static constexpr int THREADS = 64 * NW;
     static constexpr int BM = 256;
     static constexpr int BG = 128;
     static constexpr int NT = I / BG;
-    static constexpr int A_BYTES = BM * BLK;
     static constexpr int B_BYTES = 2 * BG * BLK;
-    static constexpr int SA_BYTES = BM * 4;
-    static constexpr int STAGE = A_BYTES + B_BYTES + SA_BYTES;
-    static constexpr int A_LD = A_BYTES / 1024 / NW;
-    static constexpr int B_LD = B_BYTES / 1024 / NW;
-    static_assert(A_LD == 4 && B_LD == 4, "loader split: vmcnt(4) leaves one k-block of weight copies");
-    static_assert(2 * STAGE + 2 * 64 * 4 <= 160 * 1024, "LDS budget");
+    // stage: activation rows | weight rows | row scales
+    static constexpr int A_BYTES = BM * BLK;
+    static constexpr int STAGE = A_BYTES + B_BYTES + BM * 4;
+    static constexpr int A2_BYTES = 128 * BLK;  // tiles of at most 128 rows
+    static constexpr int STAGE2 = A2_BYTES + B_BYTES + 128 * 4;
+    static constexpr int SMEM = 2 * STAGE > 3 * STAGE2 ? 2 * STAGE : 3 * STAGE2;
+    static constexpr int LAG = 3;
+    static_assert(SMEM + 2 * 64 * 4 <= 160 * 1024, "LDS budget");
     static_assert(HB <= 64 && HB >= 2, "weight scales: one lane per k-block");
 };
 
+// End of a phase: this wave's LDS reads are done and at most N of its copies
+// are outstanding; then the workgroup's barrier.
+template <int N>
+__device__ __forceinline__ void phase_end() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void phase_end() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 template <int GM>
-__global__ __launch_bounds__(512) void gemm1_tile_w_kernel(
+__global__ __launch_bounds__(512) void gemm1_tile_p_kernel(
     Plan p, const uint8_t* __restrict__ hs, const float* __restrict__ hs_scale,
     const uint8_t* __restrict__ w1, const float* __restrict__ w1s) {
-    using C = G1W;
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * C::STAGE];
+    using C = G1P;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[C::SMEM];
     __shared__ __attribute__((aligned(16))) float s_sb[2 * 64];  // [gate | up][kb] weight scales
 
     int e, row0, nrows, nt;
@@ -455,225 +478,313 @@ __global__ __launch_bounds__(512) void gemm1_tile_w_kernel(
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave & 3, wm = wave >> 2;
+    const int r = lane & 15, g = lane >> 4;
     const int jb = nt * C::BG;
+    const bool small = nrows <= 128;
 
-    uint32_t a_off[C::A_LD], b_off[C::B_LD];
+    auto token = [&](int row) __attribute__((always_inline)) {
+        return (uint32_t)p.sorted_tok[row0 + min(row, nrows - 1)];
+    };
+    uint32_t b_off[4];
 #pragma unroll
-    for (int i = 0; i < C::A_LD; ++i) {
-        const int row = 8 * (wave * C::A_LD + i) + (lane >> 3);
-        const int c = (lane & 7) ^ swzq(row);
-        const int tok = p.sorted_tok[row0 + min(row, nrows - 1)];
-        a_off[i] = (uint32_t)tok * H + c * 16;
-    }
-#pragma unroll
-    for (int i = 0; i < C::B_LD; ++i) {
-        const int row = 8 * (wave * C::B_LD + i) + (lane >> 3);
+    for (int i = 0; i < 4; ++i) {
+        const int row = 8 * (wave * 4 + i) + (lane >> 3);
         const int c = (lane & 7) ^ swzq(row);
         const int wrow = row < C::BG ? jb + row : I + jb + (row - C::BG);
         b_off[i] = (uint32_t)((e * N1 + wrow) * H + c * 16);
     }
-    // Activation scales sit in LDS as [row group wm][r][m] (row 128wm + 16m
-    // + r), so a lane reads the scales of its 8 rows as two 16-byte vectors.
-    // Waves 0..3 copy 64 of them each; lane l of wave w takes index 64w + l.
-    uint32_t sa_off = 0;
-    if (wave < 4) {
-        const int idx = 64 * wave + lane;
-        const int row = 128 * (idx >> 7) + 16 * (idx & 7) + ((idx & 127) >> 3);
-        sa_off = (uint32_t)p.sorted_tok[row0 + min(row, nrows - 1)];
-    }
-
     // copies address their rows as a k-block base (SGPRs) + a 32-bit offset
-    auto issue_a = [&](int stage, int kb) __attribute__((always_inline)) {
-        uint8_t* s = smem + stage * C::STAGE;
-        const uint8_t* base = hs + kb * BLK;
+    auto issue_b = [&](uint8_t* dst, int k) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < C::A_LD; ++i) g2l16s(base, a_off[i], s + (wave * C::A_LD + i) * 1024);
-        if (wave < 4) g2l4s(hs_scale + (size_t)kb * p.T, sa_off * 4, s + C::A_BYTES + C::B_BYTES + wave * 256);
+        for (int i = 0; i < 4; ++i) g2l16s(w1 + k * BLK, b_off[i], dst + (wave * 4 + i) * 1024);
     };
-    auto issue_b = [&](int stage, int kb) __attribute__((always_inline)) {
-        uint8_t* s = smem + stage * C::STAGE + C::A_BYTES;
-        const uint8_t* base = w1 + kb * BLK;
-#pragma unroll
-        for (int i = 0; i < C::B_LD; ++i) g2l16s(base, b_off[i], s + (wave * C::B_LD + i) * 1024);
-    };
-
     // The tile's weight scales (one 128-column block of gate, one of up, for
     // every k-block) are copied once by waves 4 and 5.
     if (wave == 4 || wave == 5) {
         const int nb = wave == 4 ? jb / BLK : (I + jb) / BLK;
         if (lane < HB) g2l4s(w1s + ((size_t)e * N1B + nb) * HB, lane * 4, s_sb + (wave - 4) * 64);
     }
-    // Prologue, in the order of the steady state: weights and activations of
-    // k-block 0, weights of 1; then (after the barrier that plays barrier Y
-    // of k-block -1) activations of 1.
-    issue_b(0, 0);
-    issue_a(0, 0);
-    issue_b(1, 1);
-    asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");
-    issue_a(1, 1);
 
-    const int wn = wave & 3, wm = wave >> 2;
-    const int r = lane & 15, g = lane >> 4;
-    const bool active = wm * 128 < nrows;  // wave-uniform: rows past the expert only copy
-
-    auto frag = [&](const uint8_t* s, int row) __attribute__((always_inline)) {
-        const uint8_t* base = s + row * BLK;
-        const int sw = swzq(row);
-        const v4i lo = lds16(base + ((g ^ sw) << 4));
-        const v4i hi = lds16(base + (((g + 4) ^ sw) << 4));
+    // fragment of 16 rows at s: this lane's row r, 16-byte chunks g and g + 4
+    const int lo_off = r * BLK + ((g ^ swzq(r)) << 4), hi_off = r * BLK + (((g + 4) ^ swzq(r)) << 4);
+    auto frag = [&](const uint8_t* s) __attribute__((always_inline)) {
+        const v4i lo = lds16(s + lo_off);
+        const v4i hi = lds16(s + hi_off);
         return (v8i){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
     };
-    auto brow = [&](int n) __attribute__((always_inline)) {
-        return n < 2 ? 32 * wn + 16 * n + r : C::BG + 32 * wn + 16 * (n - 2) + r;
+    // weight rows of column tile n (0, 1 gate; 2, 3 up) in a stage's weight region
+    auto bcol = [&](int n) __attribute__((always_inline)) {
+        return (n < 2 ? 32 * wn + 16 * n : C::BG + 32 * wn + 16 * (n - 2)) * BLK;
+    };
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+    v8i bfr[4], afr[4];   // fragments of the phase: weights, four row tiles
+    float ug[4], uu[4];   // sa * sb of this lane's rows for the gate and up columns
+    v4f pr[16];
+    auto scale4 = [&](v4f& a, int t) __attribute__((always_inline)) {
+        const float u = (t & 3) < 2 ? ug[t >> 2] : uu[t >> 2];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) a[v] += pr[t][v] * u;
+    };
+    auto factors = [&](const float4& sa, float sbg, float sbu) __attribute__((always_inline)) {
+        const float s4[4] = {sa.x, sa.y, sa.z, sa.w};
+#pragma unroll
+        for (int m = 0; m < 4; ++m) { ug[m] = s4[m] * sbg; uu[m] = s4[m] * sbu; }
+    };
+    // C phase: 16 MFMAs into acc[0..3] and the scale FMAs of all but the last
+    // LAG. Empty asm statements keep the compiler from sinking those MFMAs
+    // below the barrier.
+    auto multiply = [&](v4f (*acc)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            pr[t] = mfma_f8_16x16x128(bfr[t & 3], afr[t >> 2], zero);
+            if (t >= C::LAG) scale4(acc[(t - C::LAG) >> 2][(t - C::LAG) & 3], t - C::LAG);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int t = 16 - C::LAG; t < 16; ++t) asm volatile("" : "+v"(pr[t]));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // the last LAG scale FMAs of the phase before
+    auto finish = [&](v4f (*acc)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 16 - C::LAG; t < 16; ++t) scale4(acc[t >> 2][t & 3], t);
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            asm volatile("" : "+v"(acc[m][0]), "+v"(acc[m][1]), "+v"(acc[m][2]), "+v"(acc[m][3]));
+    };
+    auto store_row = [&](int row, const v4f (&a)[4]) __attribute__((always_inline)) {
+        if (row >= nrows) return;
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            uint32_t w[2], wl[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float v0 = silu(a[n + 2][2 * h]) * a[n][2 * h];
+                const float v1 = silu(a[n + 2][2 * h + 1]) * a[n][2 * h + 1];
+                const uint16_t h0 = f2bf(v0), h1 = f2bf(v1);
+                w[h] = (uint32_t)h0 | ((uint32_t)h1 << 16);
+                wl[h] = (uint32_t)f2bf(v0 - bf2f(h0)) | ((uint32_t)f2bf(v1 - bf2f(h1)) << 16);
+            }
+            const size_t idx = (size_t)(row0 + row) * I + jb + wn * 32 + n * 16 + 4 * g;
+            *reinterpret_cast<uint2*>(p.act + idx) = make_uint2(w[0], w[1]);
+            if (p.act_lo) *reinterpret_cast<uint2*>(p.act_lo + idx) = make_uint2(wl[0], wl[1]);
+        }
     };
 
-    if (!active) {
-        // Rows past the expert: copies and barriers only, in step with the
-        // other waves (two barriers per k-block).
-#pragma unroll 1
-        for (int kb = 0; kb < HB; ++kb) {
-            const int kb2 = min(kb + 2, HB - 1);
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            issue_b(kb & 1, kb2);
-            asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            issue_a(kb & 1, kb2);
-        }
-        wait_vmem();  // no copy into LDS may be pending when the workgroup ends
-        return;
-    }
-
-    // The arithmetic of one wave with MT row tiles (8, or 4 when the wave's
-    // rows past 64 lie beyond the expert: partial row tiles at the end of an
-    // expert then cost half the MFMAs). Both forms run the same copies and
-    // barriers.
-    auto compute = [&](auto mt_c) __attribute__((always_inline)) {
+    // A tile of more than 128 rows. G: the wave's group; MT: its row tiles
+    // that are multiplied (8; 4 when its rows past 64 lie beyond the expert).
+    auto large_tile = [&](auto g_c, auto mt_c) __attribute__((always_inline)) {
+        constexpr int G = decltype(g_c)::value;
         constexpr int MT = decltype(mt_c)::value;
-        static_assert(MT >= 3 && MT <= 8, "barrier X after row tile 0, Y before the last");
-        constexpr int NTT = 4 * MT;        // MFMAs per k-block
-        constexpr int TY = 4 * (MT - 1);   // barrier Y before the last row tile
-        // scale factors sa * sb of this lane's rows (128wm + 16m + r) for the
-        // gate and up column blocks of k-block kb (stage s)
-        float ug[MT], uu[MT];
-        auto scales = [&](const uint8_t* s, int kb) __attribute__((always_inline)) {
-            const float* sSA = reinterpret_cast<const float*>(s + C::A_BYTES + C::B_BYTES);
-            const float4 s0 = *reinterpret_cast<const float4*>(sSA + wm * 128 + r * 8);
-            const float4 s1 = *reinterpret_cast<const float4*>(sSA + wm * 128 + r * 8 + 4);
-            const float sa[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-            const float sbg = s_sb[kb], sbu = s_sb[64 + kb];
+        constexpr int NV = 4 + 2 + (G == 0) + 2;  // weights, rows, group 0's row scales, rows
+        // activation halves: rows 0-63 and 128-191 (row tiles 0-3 of both
+        // groups), rows 64-127 and 192-255
+        uint32_t a_off[4];
 #pragma unroll
-            for (int m = 0; m < MT; ++m) { ug[m] = sa[m] * sbg; uu[m] = sa[m] * sbu; }
+        for (int i = 0; i < 4; ++i) {
+            const int j = wave * 2 + (i & 1);
+            const int row = (i >> 1) * 64 + (j >> 3) * 128 + (j & 7) * 8 + (lane >> 3);
+            a_off[i] = token(row) * H + ((lane & 7) ^ swzq(row)) * 16;
+        }
+        // row scales sit in LDS as [row group][r][m] (row 128wm + 16m + r), so
+        // a lane reads those of its 8 rows as two 16-byte vectors; wave w of
+        // group 0 copies 64 of them
+        uint32_t sa_off = 0;
+        if constexpr (G == 0) {
+            const int idx = 64 * wave + lane;
+            sa_off = token(128 * (idx >> 7) + 16 * (idx & 7) + ((idx & 127) >> 3)) * 4;
+        }
+        auto issue_a = [&](int half, int kb) __attribute__((always_inline)) {
+            uint8_t* s = smem + (kb & 1) * C::STAGE;
+            const uint8_t* base = hs + min(kb, HB - 1) * BLK;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int j = wave * 2 + i;
+                g2l16s(base, a_off[half * 2 + i], s + (half * 64 + (j >> 3) * 128 + (j & 7) * 8) * BLK);
+            }
         };
+        auto issue_ba = [&](int kb) __attribute__((always_inline)) {
+            uint8_t* s = smem + (kb & 1) * C::STAGE + C::A_BYTES;
+            const int k = min(kb, HB - 1);
+            issue_b(s, k);
+            issue_a(0, kb);
+            if constexpr (G == 0) g2l4s(hs_scale + (size_t)k * p.T, sa_off, s + C::B_BYTES + wave * 256);
+        };
+        issue_ba(0);
+        issue_a(1, 0);
+        issue_ba(1);
+        phase_end<NV>();
+        if constexpr (G == 1) phase_end();
 
-        v4f acc[MT][4];  // [row tile m][column tile n: 0, 1 gate; 2, 3 up]
-        const v4f zero = {0.f, 0.f, 0.f, 0.f};
+        v4f acc[8][4];
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (int n = 0; n < 4; ++n) acc[m][n] = zero;
-        // weight fragments of the k-block; activation fragments of the current
-        // row tile and the next two (each read two row tiles ahead of its
-        // MFMAs: one row tile of MFMAs is shorter than an LDS read under load)
-        v8i bfr[4], acur, anx1, anx2;
-#pragma unroll
-        for (int n = 0; n < 4; ++n) bfr[n] = frag(smem + C::A_BYTES, brow(n));
-        acur = frag(smem, wm * 128 + r);
-        anx1 = frag(smem, wm * 128 + 16 + r);
-        scales(smem, 0);
-
-        // The k-loop is straight-line code: the copies of the last two
-        // k-blocks repeat k-block HB-1 into regions no wave reads again, and
-        // the fragments and scales read for "k-block HB" are never used.
+        // The copies of k-blocks past the last repeat it into regions that no
+        // wave reads again.
 #pragma unroll 1
         for (int kb = 0; kb < HB; ++kb) {
-            const int cur = kb & 1;
-            uint8_t* const sc = smem + cur * C::STAGE;        // this k-block's stage
-            uint8_t* const sn = smem + (cur ^ 1) * C::STAGE;  // the next one's
-            const int kb1 = min(kb + 1, HB - 1), kb2 = min(kb + 2, HB - 1);
-            // scale-and-accumulate of MFMA result x (row tile tm, column tile tn)
-            auto fma4 = [&](const v4f& x, int tm, int tn) __attribute__((always_inline)) {
-                const float u = tn < 2 ? ug[tm] : uu[tm];
+            const uint8_t* st = smem + (kb & 1) * C::STAGE;
+            const uint8_t* sA = st + wm * 128 * BLK;
+            const float* sSA = reinterpret_cast<const float*>(st + C::A_BYTES + C::B_BYTES) + wm * 128 + r * 8;
+            // M0
 #pragma unroll
-                for (int v = 0; v < 4; ++v) acc[tm][tn][v] += x[v] * u;
-            };
-            // The compiler would sink the MFMAs and FMAs below the barriers
-            // (they touch no memory) and hoist all fragment reads to the top,
-            // keeping every fragment live at once: empty asm statements naming
-            // the accumulators pin the arithmetic before each barrier, and a
-            // compiler-only memory fence per row tile keeps each activation
-            // fragment read in its row tile.
-            auto pin_rows = [&](int m0, int m1) __attribute__((always_inline)) {
+            for (int n = 0; n < 4; ++n) bfr[n] = frag(st + C::A_BYTES + bcol(n));
 #pragma unroll
-                for (int m = m0; m < m1; ++m)
-                    asm volatile("" : "+v"(acc[m][0]), "+v"(acc[m][1]), "+v"(acc[m][2]), "+v"(acc[m][3]));
-            };
-            v4f pr[NTT];
+            for (int m = 0; m < 4; ++m) afr[m] = frag(sA + m * 16 * BLK);
+            const float4 sa0 = *reinterpret_cast<const float4*>(sSA);
+            // read here, not in M1: group 0 copies kb + 2's scales over them there
+            float4 sa1 = sa0;
+            if constexpr (MT > 4) sa1 = *reinterpret_cast<const float4*>(sSA + 4);
+            const float sbg = s_sb[kb], sbu = s_sb[64 + kb];
+            __builtin_amdgcn_sched_barrier(0);
+            issue_a(1, kb + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (MT > 4) {
+                if (kb) finish(acc + 4);
+            }
+            factors(sa0, sbg, sbu);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (G == 1) phase_end<NV>(); else phase_end();
+            // C0
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(acc);
+            if constexpr (G == 0) phase_end<NV>(); else phase_end();
+            // M1
+            if constexpr (MT > 4) {
 #pragma unroll
-            for (int t = 0; t < NTT; ++t) {
-                const int m = t >> 2, n = t & 3;
-                if (n == 0) asm volatile("" ::: "memory");
-                if (t == 4) {  // barrier X: weight fragments of kb are in registers everywhere
-                    pin_rows(MT - 2, MT);
-                    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                    issue_b(cur, kb2);
-                }
-                if (t == TY) {  // barrier Y: k-block kb+1 has landed; activations of kb all read
-                    pin_rows(0, MT - 2);
-                    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                    issue_a(cur, kb2);
-                }
-                // activation fragments two row tiles ahead: rows of kb while
-                // m < MT - 2; the first two row tiles of kb+1 once it has landed
-                if (n == 0 && m < MT - 2) anx2 = frag(sc, wm * 128 + 16 * (m + 2) + r);
-                if (t == TY) anx1 = frag(sn, wm * 128 + r);
-                if (t == TY + 1) anx2 = frag(sn, wm * 128 + 16 + r);
-                pr[t] = mfma_f8_16x16x128(bfr[n], acur, zero);
-                if (m == MT - 1) bfr[n] = frag(sn + C::A_BYTES, brow(n));
-                if (n == 3) {  // the next row tile's fragment becomes current
-                    acur = anx1;
-                    anx1 = anx2;
-                }
-                if (t >= 4) fma4(pr[t - 4], (t - 4) >> 2, (t - 4) & 3);
+                for (int m = 0; m < 4; ++m) afr[m] = frag(sA + (64 + m * 16) * BLK);
                 __builtin_amdgcn_sched_barrier(0);
             }
-#pragma unroll
-            for (int n = 0; n < 4; ++n) fma4(pr[NTT - 4 + n], MT - 1, n);
-            scales(sn, kb1);
-        }
-        wait_vmem();  // no copy into LDS may be pending when the workgroup ends
-
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const int row = wm * 128 + m * 16 + r;
-            if (row < nrows) {
-#pragma unroll
-                for (int n = 0; n < 2; ++n) {
-                    uint32_t w[2], wl[2];
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const float v0 = silu(acc[m][n + 2][2 * h]) * acc[m][n][2 * h];
-                        const float v1 = silu(acc[m][n + 2][2 * h + 1]) * acc[m][n][2 * h + 1];
-                        const uint16_t h0 = f2bf(v0), h1 = f2bf(v1);
-                        w[h] = (uint32_t)h0 | ((uint32_t)h1 << 16);
-                        wl[h] = (uint32_t)f2bf(v0 - bf2f(h0)) | ((uint32_t)f2bf(v1 - bf2f(h1)) << 16);
-                    }
-                    const size_t idx = (size_t)(row0 + row) * I + jb + wn * 32 + n * 16 + 4 * g;
-                    *reinterpret_cast<uint2*>(p.act + idx) = make_uint2(w[0], w[1]);
-                    if (p.act_lo) *reinterpret_cast<uint2*>(p.act_lo + idx) = make_uint2(wl[0], wl[1]);
-                }
+            issue_ba(kb + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            finish(acc);
+            if constexpr (MT > 4) factors(sa1, sbg, sbu);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (G == 1) phase_end<NV>(); else phase_end();
+            // C1
+            if constexpr (MT > 4) {
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(acc + 4);
             }
+            if constexpr (G == 0) phase_end<NV>(); else phase_end();
+        }
+        if constexpr (MT > 4) finish(acc + 4);
+        if constexpr (G == 0) phase_end();
+        wait_vmem();  // no copy into LDS may be pending when the workgroup ends
+#pragma unroll
+        for (int m = 0; m < MT; ++m) store_row(wm * 128 + m * 16 + r, acc[m]);
+    };
+
+    // A tile of at most 128 rows: group wm takes rows 64wm .. 64wm+63, two
+    // phases a k-block, three stages. Rows past the expert (ACTIVE false) only
+    // copy, in step with the others.
+    auto small_tile = [&](auto g_c, auto active_c) __attribute__((always_inline)) {
+        constexpr int G = decltype(g_c)::value;
+        constexpr bool ACTIVE = decltype(active_c)::value;
+        constexpr int NV = 4 + 2 + (G == 0);
+        uint32_t a_off[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int row = (wave * 2 + i) * 8 + (lane >> 3);
+            a_off[i] = token(row) * H + ((lane & 7) ^ swzq(row)) * 16;
+        }
+        // row scales as [row group][r][m] (row 64wm + 16m + r); waves 2 and 3
+        // repeat the copies of waves 0 and 1, so that a group's waves count alike
+        uint32_t sa_off = 0;
+        if constexpr (G == 0) {
+            const int idx = 64 * (wave & 1) + lane;
+            sa_off = token(64 * (idx >> 6) + 16 * (idx & 3) + ((idx & 63) >> 2)) * 4;
+        }
+        auto issue = [&](int so, int kb) __attribute__((always_inline)) {
+            uint8_t* s = smem + so;
+            const int k = min(kb, HB - 1);
+            issue_b(s + C::A2_BYTES, k);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) g2l16s(hs + k * BLK, a_off[i], s + (wave * 2 + i) * 1024);
+            if constexpr (G == 0)
+                g2l4s(hs_scale + (size_t)k * p.T, sa_off, s + C::A2_BYTES + C::B_BYTES + (wave & 1) * 256);
+        };
+        issue(0, 0);
+        issue(C::STAGE2, 1);
+        phase_end<NV>();
+        if constexpr (G == 1) phase_end();
+
+        v4f acc[4][4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) acc[m][n] = zero;
+        int s0 = 0, s2 = 2 * C::STAGE2;  // stages of kb and kb + 2
+#pragma unroll 1
+        for (int kb = 0; kb < HB; ++kb) {
+            const uint8_t* st = smem + s0;
+            // M
+            float4 sa;
+            float sbg, sbu;
+            if constexpr (ACTIVE) {
+#pragma unroll
+                for (int n = 0; n < 4; ++n) bfr[n] = frag(st + C::A2_BYTES + bcol(n));
+#pragma unroll
+                for (int m = 0; m < 4; ++m) afr[m] = frag(st + (wm * 64 + m * 16) * BLK);
+                sa = *reinterpret_cast<const float4*>(
+                    reinterpret_cast<const float*>(st + C::A2_BYTES + C::B_BYTES) + wm * 64 + r * 4);
+                sbg = s_sb[kb];
+                sbu = s_sb[64 + kb];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            issue(s2, kb + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (ACTIVE) {
+                if (kb) finish(acc);
+                factors(sa, sbg, sbu);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (G == 1) phase_end<NV>(); else phase_end();
+            // C
+            if constexpr (ACTIVE) {
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(acc);
+            }
+            if constexpr (G == 0) phase_end<NV>(); else phase_end();
+            s0 = s0 == 2 * C::STAGE2 ? 0 : s0 + C::STAGE2;
+            s2 = s2 == 2 * C::STAGE2 ? 0 : s2 + C::STAGE2;
+        }
+        if constexpr (ACTIVE) finish(acc);
+        if constexpr (G == 0) phase_end();
+        wait_vmem();  // no copy into LDS may be pending when the workgroup ends
+        if constexpr (ACTIVE) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) store_row(wm * 64 + m * 16 + r, acc[m]);
         }
     };
-    if (nrows - wm * 128 > 64)
-        compute(IntC<8>{});
-    else
-        compute(IntC<4>{});
+
+    if (small) {
+        if (wm == 0)
+            small_tile(IntC<0>{}, BoolC<true>{});
+        else if (nrows > 64)
+            small_tile(IntC<1>{}, BoolC<true>{});
+        else
+            small_tile(IntC<1>{}, BoolC<false>{});
+    } else if (wm == 0) {
+        large_tile(IntC<0>{}, IntC<8>{});
+    } else if (nrows > 192) {
+        large_tile(IntC<1>{}, IntC<8>{});
+    } else {
+        large_tile(IntC<1>{}, IntC<4>{});
+    }
 }
 
 hipError_t launch_gemm1_tile(const Plan& p, const uint8_t* hs, const float* hs_scale,
                              const uint8_t* w1, const float* w1s, int variant, hipStream_t s) {
     if (variant == 19) {
-        const int tiles = max_mtiles(p.T, G1W::BM) * G1W::NT;
-        hipLaunchKernelGGL((gemm1_tile_w_kernel<16>), dim3((tiles + 7) / 8 * 8), dim3(G1W::THREADS), 0,
+        // 8 row tiles per XCD walk: with 16, 2 columns x 16 rows of tiles run at
+        // a time and copy 1.5x the distinct lines of 4 x 8 (T=14000 with every
+        // token on 8 experts 2,755 against 2,705 us; T=8192 level).
+        const int tiles = max_mtiles(p.T, G1P::BM) * G1P::NT;
+        hipLaunchKernelGGL((gemm1_tile_p_kernel<8>), dim3((tiles + 7) / 8 * 8), dim3(G1P::THREADS), 0,
                            s, p, hs, hs_scale, w1, w1s);
     } else if (variant == 18) {
         using C = G1Tile<4, 2>;

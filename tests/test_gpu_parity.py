@@ -450,7 +450,7 @@ def test_every_gemm_variant_matches_oracle(name, variant, monkeypatch):
 @pytest.mark.parametrize("name", ["c3_t8192", "c4_t14000_skew"])
 def test_wide_variants_large(name, variant, monkeypatch):
     """The wide kernels and the LDS tiles (GEMM1 variant 3, 18 with swapped
-    operands, 19 with register-held weight fragments; GEMM2 variant 3, its
+    operands, 19 with two wave groups taking turns; GEMM2 variant 3, its
     pipelined form 20 and that form run by one workgroup per CU, 21) at prefill sizes: many row tiles per expert (T=8192)
     and 14,000 rows on each of 8 experts."""
     log(f"test_wide_variants_large[{name}-{variant}]")
@@ -459,6 +459,27 @@ def test_wide_variants_large(name, variant, monkeypatch):
     out = run_gpu(wl, fill=float("nan"))
     assert torch.isfinite(out.float()).all()
     _check_output(wl, out, spread_tokens(wl.T, 48))
+
+
+# Rows per expert around what GEMM1's tile does differently: 64 rows a wave group
+# in tiles of at most 128 rows, then 4 or 8 row tiles in the second group, then
+# a second row tile of either form.
+@pytest.mark.parametrize("T", [1, 16, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 384,
+                               385, 449])
+@pytest.mark.parametrize("shape", [(7168, 2048), (4096, 1536)])
+def test_gemm1_tile_row_edges(shape, T, monkeypatch):
+    """Every token on the same 8 experts, T rows each: GEMM1's two-group tile
+    (variant 19) gives the bits of the plain LDS tile (3), whose products and
+    order of sums it keeps, and the oracle's values."""
+    log(f"test_gemm1_tile_row_edges[{shape}:{T}]")
+    wl = W.make_workload(f"rows_{T}", T=T, seed=4000 + T, skew=True, H=shape[0], I=shape[1])
+    monkeypatch.setenv("MI_MOE_VARIANT", "3,3")
+    plain = run_gpu(wl, fill=float("nan")).clone()
+    monkeypatch.setenv("MI_MOE_VARIANT", "19,3")
+    out = run_gpu(wl, fill=float("nan"))
+    assert torch.equal(out.view(torch.int16), plain.view(torch.int16))
+    if T in (64, 129, 449):
+        _check_output(wl, out, spread_tokens(T, 8))
 
 
 @pytest.mark.parametrize("name,T,variant", [
