@@ -223,18 +223,26 @@ __device__ __forceinline__ int lane_id() { return __lane_id(); }
 __device__ __forceinline__ v4i ld16(const void* p) { return *reinterpret_cast<const v4i*>(p); }
 
 // Weight operand of one 16-row x 128-byte k-block, read as whole lines.
-// Lane l (n = l % 16, q = l / 16) loads 16 bytes at wl_off from row n % 8
-// (x) and from row 8 + n % 8 (y), bytes [32q + 16(n / 8), +16): each load
+// Lane l (m = (l / 2) % 8, q = l / 16) loads 16 bytes at wl_off from row 2m
+// (x) and from row 2m + 1 (y), bytes [32q + 16(l % 2), +16): each load
 // instruction covers 8 complete 128-byte lines, which non-temporal loads
 // stream from HBM about 15% faster than the 16 half lines of a row-per-lane
 // layout (measured on MI355X: 7.1 against 6.2 TB/s plain, and 5.7 TB/s for
-// half lines with the non-temporal hint). Rotating each 16-lane row by 8
-// (DPP; lanes 8-15 take y of lane n - 8, lanes 0-7 x of lane n + 8) leaves
-// lane l with row n, bytes [32q, 32q + 32): the MFMA operand in its own k
-// order, which the activation side reads with ld_afrag (fp8) or as 32
-// consecutive bf16.
+// half lines with the non-temporal hint). Exchanging x and y between the two
+// lanes of a pair (wl_frag) leaves lane l with row n = l % 16, bytes
+// [32q, 32q + 32): the MFMA operand in its own k order, in which the
+// activation side is read too (ld_araw).
+//
+// The pair matters: the address unit takes a contiguous run of lanes per
+// clock, so neighbouring lanes in different rows move 16 bytes a clock and CU
+// whatever cache answers (9.7 TB/s over the card from L2; 19 TB/s by pairs, 30
+// by fours, which would take 2.5 times the exchange). Weights and activations
+// together ran into that in every streaming kernel: T=64 GEMM1 moved 0.88 GB
+// through it, 91 us at 9.7 TB/s. Per call, one process each, weights by pairs
+// against lanes 8 rows apart: T=1 28.7 against 31.7 us, T=4 47.1 / 50.9, T=16
+// 61.0 / 64.8, T=64 87.5 / 93.0.
 __device__ __forceinline__ size_t wl_off(int lane, size_t row_stride) {
-    return (size_t)(lane & 7) * row_stride + (lane >> 4) * 32 + ((lane >> 3) & 1) * 16;
+    return (size_t)(lane & 14) * row_stride + (lane >> 4) * 32 + (lane & 1) * 16;
 }
 
 // Buffer resource over `bytes` bytes at a uniform `base`: raw buffer loads
@@ -244,27 +252,28 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t wrsrc(const void* base, uint32
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
 }
 
-// The two loads of a weight k-block (off = row base + wl_off, stride8 = 8
-// rows), kept raw in a prefetch ring: the exchange (wl_frag) runs where the
+// The two loads of a weight k-block (off = row base + wl_off, stride = one
+// row), kept raw in a prefetch ring: the exchange (wl_frag) runs where the
 // operand is consumed, so the loads stay in flight until then.
 // NT: non-temporal loads. They stream weights that no other row tile of the
 // launch reads again ~12 % faster; where several row tiles of an expert
 // re-read its weights, plain loads keep them in L2 / MALL for the others
 // (with the hint each tile fetched them from HBM again: T=1024 with up to 8
 // row tiles per expert, GEMM1 564 against 475 us). The policy is a template
-// argument: per workgroup from its expert's row count in the wide GEMM1 and
-// the stream GEMM2 (two copies of the k loop, BoolC below); per launch from
-// T (wt_nt) in the stream GEMM1, whose two-copy form took 69 -> 96 VGPRs
-// (108 without the sort folded in), and in the GEMM2 + combine kernel.
+// argument: per workgroup from its expert's row count in the wide GEMM1, the
+// stream GEMM2 and the stream GEMM1's front forms (two copies of the k loop,
+// BoolC below; T=64 with every token on 8 experts, four 16-row tiles each:
+// GEMM1 102 against 135 us with the hint); per launch from T (wt_nt) in the
+// other stream GEMM1 forms and in the GEMM2 + combine kernel.
 struct WRaw {
     v4i x, y;
 };
 template <bool NT>
-__device__ __forceinline__ WRaw ld_wraw(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t stride8) {
+__device__ __forceinline__ WRaw ld_wraw(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t stride) {
     constexpr int AUX = NT ? 2 : 0;  // cache policy: nt
     WRaw w;
     w.x = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, AUX));
-    w.y = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off + stride8), 0, AUX));
+    w.y = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off + stride), 0, AUX));
     return w;
 }
 
@@ -291,28 +300,48 @@ struct IntC {
 };
 
 __device__ __forceinline__ v8i wl_frag(const WRaw& w) {
-    constexpr int ROR8 = 0x128;  // DPP row_ror:8
+    constexpr int SWAP = 0xB1;  // DPP quad_perm [1, 0, 3, 2]: the pair's other lane
+    const bool even = (__lane_id() & 1) == 0;
     v8i r;
-    r.s0 = __builtin_amdgcn_update_dpp(w.x.x, w.y.x, ROR8, 0xF, 0xC, false);
-    r.s1 = __builtin_amdgcn_update_dpp(w.x.y, w.y.y, ROR8, 0xF, 0xC, false);
-    r.s2 = __builtin_amdgcn_update_dpp(w.x.z, w.y.z, ROR8, 0xF, 0xC, false);
-    r.s3 = __builtin_amdgcn_update_dpp(w.x.w, w.y.w, ROR8, 0xF, 0xC, false);
-    r.s4 = __builtin_amdgcn_update_dpp(w.y.x, w.x.x, ROR8, 0xF, 0x3, false);
-    r.s5 = __builtin_amdgcn_update_dpp(w.y.y, w.x.y, ROR8, 0xF, 0x3, false);
-    r.s6 = __builtin_amdgcn_update_dpp(w.y.z, w.x.z, ROR8, 0xF, 0x3, false);
-    r.s7 = __builtin_amdgcn_update_dpp(w.y.w, w.x.w, ROR8, 0xF, 0x3, false);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int xs = __builtin_amdgcn_mov_dpp(w.x[i], SWAP, 0xF, 0xF, true);
+        const int ys = __builtin_amdgcn_mov_dpp(w.y[i], SWAP, 0xF, 0xF, true);
+        r[i] = even ? w.x[i] : ys;
+        r[4 + i] = even ? xs : w.y[i];
+    }
     return r;
 }
 
-// The fp8 activation operand matching wl_frag: bytes [32q, 32q + 32) of the
-// k-block (p = row + k-block + 32q).
-__device__ __forceinline__ v8i ld_afrag(const uint8_t* p) {
-    const v4i lo = ld16(p);
-    const v4i hi = ld16(p + 16);
-    v8i r;
-    r.s0 = lo.x; r.s1 = lo.y; r.s2 = lo.z; r.s3 = lo.w;
-    r.s4 = hi.x; r.s5 = hi.y; r.s6 = hi.z; r.s7 = hi.w;
-    return r;
+// The activation operand in the same k order: 16 bytes at off0 and 16 at off1
+// (+ k) per lane. PAIR: as the weights, a pair's lanes load 16 bytes each of
+// both its rows, 2m and 2m + 1, and exchange them in a_frag; for row tiles with
+// many rows, whose expert has more than one. Without, a lane loads the 32
+// bytes of its own row: what tiles of a few rows do, whose lanes past them
+// repeat a row (with PAIR T = 1 ... 37 2 us slower per call, T=64 1 % faster).
+template <bool PAIR>
+__device__ __forceinline__ void a_offs(int lane, uint32_t own_row, int bytes_per_lane, uint32_t (&off)[2]) {
+    const uint32_t k = (lane >> 4) * bytes_per_lane;
+    if constexpr (PAIR) {
+        const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)own_row, 0xB1, 0xF, 0xF, true);
+        off[0] = (lane & 1 ? other : own_row) + k + (lane & 1) * 16;
+        off[1] = (lane & 1 ? own_row : other) + k + (lane & 1) * 16;
+    } else {
+        off[0] = own_row + k;
+        off[1] = own_row + k + 16;
+    }
+}
+__device__ __forceinline__ WRaw ld_araw(const void* base, const uint32_t (&off)[2], int k) {
+    const uint8_t* b = reinterpret_cast<const uint8_t*>(base) + k;
+    WRaw w;
+    w.x = *reinterpret_cast<const v4i*>(b + off[0]);
+    w.y = *reinterpret_cast<const v4i*>(b + off[1]);
+    return w;
+}
+template <bool PAIR>
+__device__ __forceinline__ v8i a_frag(const WRaw& w) {
+    if constexpr (PAIR) return wl_frag(w);
+    return (v8i){w.x.x, w.x.y, w.x.z, w.x.w, w.y.x, w.y.y, w.y.z, w.y.w};
 }
 
 // A token's top-k row in a TOPK_LD-strided table (workspace or LDS, 16-byte

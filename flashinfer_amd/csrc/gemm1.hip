@@ -20,9 +20,9 @@
 //
 // Operand layout: lane l feeds row (l % 16) of a 16x128 operand with bytes
 // [32g, 32g+32) of the 128-byte k-block, g = l / 16. The weights arrive as
-// whole 128-byte lines (two non-temporal loads per k-block, exchanged within
-// 16-lane rows by wl_frag where they are consumed); the activation row is
-// read at the same k offsets (ld_afrag).
+// whole 128-byte lines (two non-temporal loads per k-block, exchanged between
+// neighbouring lanes by wl_frag where they are consumed); the activation row is
+// read at the same k offsets (ld_araw).
 //
 // With FRONT_SORT (T <= 64, MT = 1) the kernel also stands in for the sort
 // launch: each wave builds the row-tile table from the top-k ids in its
@@ -71,9 +71,12 @@ void gemm1_stream_kernel(Plan p, const uint8_t* __restrict__ hs, const float* __
     // weight columns. The lane index comes in as an argument: the tile loop
     // of the front kernels passes it through an empty asm statement, so the
     // compiler recomputes the lane's addresses per tile instead of holding
-    // them across the loop (77 instead of 96 VGPRs and spills).
-    auto tile = [&](int e, const int row0, const int nrows, const int (&tok)[MT], const int lane,
+    // them across the loop (92 VGPRs with both load policies; five waves per
+    // SIMD). nt_c: weight load policy of the tile.
+    auto tile = [&](auto nt_c, int e, const int row0, const int nrows, const int (&tok)[MT], const int lane,
                     const int col) __attribute__((always_inline)) {
+        constexpr bool WNT = decltype(nt_c)::value;
+        constexpr bool PAIR = NT && !WNT;            // more rows than one tile's
         const int r = lane & 15, g = lane >> 4;
         const int tid = wave * 64 + lane;
         const int wc = wave % NW;         // column group
@@ -84,15 +87,15 @@ void gemm1_stream_kernel(Plan p, const uint8_t* __restrict__ hs, const float* __
         const __amdgpu_buffer_rsrc_t wr = wrsrc(w1 + (size_t)e * N1 * H, (uint32_t)((size_t)N1 * H));
         const uint32_t bg_off = (uint32_t)((size_t)j0 * H + (size_t)ks * KB * BLK + wl_off(lane, H));
         const uint32_t bu_off = bg_off + (uint32_t)((size_t)I * H);
-        const uint8_t* a_ptr[MT];
+        uint32_t a_off[MT][2];
 #pragma unroll
-        for (int i = 0; i < MT; ++i) a_ptr[i] = hs + (size_t)tok[i] * H + ks * KB * BLK + g * 32;
+        for (int i = 0; i < MT; ++i) a_offs<PAIR>(lane, (uint32_t)tok[i] * H + ks * KB * BLK, 32, a_off[i]);
         const float* sbg_ptr = w1s + ((size_t)e * N1B + j0 / BLK) * HB + ks * KB;
         const float* sbu_ptr = w1s + ((size_t)e * N1B + (I + j0) / BLK) * HB + ks * KB;
         const float (*sa_k)[BM] = sa_lds + ks * KB;  // this wave's k-blocks
 
         WRaw bg[D], bu[D];
-        v8i a[D][MT];
+        WRaw a[D][MT];
         v4f accg[MT], accu[MT];
         const v4f zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -107,8 +110,9 @@ void gemm1_stream_kernel(Plan p, const uint8_t* __restrict__ hs, const float* __
             const v8i fu = wl_frag(bu[d]);
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
-                const v4f pg = mfma_f8_16x16x128(a[d][i], fg, zero);
-                const v4f pu = mfma_f8_16x16x128(a[d][i], fu, zero);
+                const v8i fa = a_frag<PAIR>(a[d][i]);
+                const v4f pg = mfma_f8_16x16x128(fa, fg, zero);
+                const v4f pu = mfma_f8_16x16x128(fa, fu, zero);
                 const float4 sa4 = *reinterpret_cast<const float4*>(&sa_k[kb][i * 16 + g * 4]);
                 accg[i][0] += pg[0] * (sa4.x * sg);
                 accg[i][1] += pg[1] * (sa4.y * sg);
@@ -122,10 +126,10 @@ void gemm1_stream_kernel(Plan p, const uint8_t* __restrict__ hs, const float* __
         };
         auto load = [&](int d, int kb) __attribute__((always_inline)) {
             const int nk = kb * BLK;
-            bg[d] = ld_wraw<NT>(wr, bg_off + nk, 8 * H);
-            bu[d] = ld_wraw<NT>(wr, bu_off + nk, 8 * H);
+            bg[d] = ld_wraw<WNT>(wr, bg_off + nk, H);
+            bu[d] = ld_wraw<WNT>(wr, bu_off + nk, H);
 #pragma unroll
-            for (int i = 0; i < MT; ++i) a[d][i] = ld_afrag(a_ptr[i] + nk);
+            for (int i = 0; i < MT; ++i) a[d][i] = ld_araw(hs, a_off[i], nk);
         };
 
         // Start streaming weights first; the activation scales of the tile go to
@@ -228,7 +232,7 @@ void gemm1_stream_kernel(Plan p, const uint8_t* __restrict__ hs, const float* __
                 if (mt != row) __syncthreads();  // the last tile's reads of sa_lds are done
                 int ln = lane;
                 asm volatile("" : "+v"(ln));
-                tile(nth_set_bit((unsigned long long)m, mt), mt, 1, tok, ln, col);
+                tile(BoolC<NT>{}, nth_set_bit((unsigned long long)m, mt), mt, 1, tok, ln, col);
             }
             return;
         }
@@ -267,7 +271,10 @@ void gemm1_stream_kernel(Plan p, const uint8_t* __restrict__ hs, const float* __
             if (mt != row) __syncthreads();  // the last tile's reads of sa_lds are done
             int ln = lane;
             asm volatile("" : "+v"(ln));
-            tile(wt.e, wt.row0, wt.nrows, tok, ln, col);
+            // An expert with more than this row tile: plain weight loads, which the
+            // other tiles find in L2, and activation rows by pairs.
+            if (NT && wt.count > BM) tile(BoolC<false>{}, wt.e, wt.row0, wt.nrows, tok, ln, col);
+            else tile(BoolC<NT>{}, wt.e, wt.row0, wt.nrows, tok, ln, col);
         }
     } else {
         int e, row0, nrows;
@@ -275,7 +282,7 @@ void gemm1_stream_kernel(Plan p, const uint8_t* __restrict__ hs, const float* __
         int tok[MT];
 #pragma unroll
         for (int i = 0; i < MT; ++i) tok[i] = p.sorted_tok[row0 + min(i * 16 + (lane & 15), nrows - 1)];
-        tile(e, row0, nrows, tok, lane, blockIdx.x);
+        tile(BoolC<NT>{}, e, row0, nrows, tok, lane, blockIdx.x);
     }
 }
 

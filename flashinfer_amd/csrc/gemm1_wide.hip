@@ -235,8 +235,8 @@ __global__ __launch_bounds__(64 * WIDE_NW) void gemm1_wide_kernel(Plan p, const 
         float sgs[DA], sus[DA];  // weight scales of the staged k-blocks (uniform)
 
         auto load_w = [&](int d, int kb) __attribute__((always_inline)) {
-            bg[d] = ld_wraw<NT>(wr, bg_off + kb * BLK, 8 * H);
-            bu[d] = ld_wraw<NT>(wr, bu_off + kb * BLK, 8 * H);
+            bg[d] = ld_wraw<NT>(wr, bg_off + kb * BLK, H);
+            bu[d] = ld_wraw<NT>(wr, bu_off + kb * BLK, H);
         };
         auto load_a = [&](int s, int kb) __attribute__((always_inline)) {
 #pragma unroll

@@ -26,7 +26,7 @@
 //
 // Operand layout: lane l (row l % 16, g = l / 16) holds bytes [32g, 32g+32)
 // of the 128-wide k-block of its weight row (whole-line non-temporal loads,
-// exchanged within 16-lane rows by wl_frag where they are consumed); MFMA h
+// exchanged between neighbouring lanes by wl_frag where they are consumed); MFMA h
 // (h = 0..3) consumes bytes [8h, 8h+8) of those 32, i.e. k-block offsets
 // 32g + 8h. The activation operand is loaded with the same k offsets, so A
 // and B always pair the same k.
@@ -38,14 +38,18 @@ struct Frag16 {
     v4i c0, c1, c2, c3;  // four 8 x bf16 operands
 };
 
-__device__ __forceinline__ Frag16 ld_act(const uint16_t* row, int kb, int g) {
-    const uint16_t* p0 = row + kb * BLK + g * 32;
-    Frag16 f;
-    f.c0 = ld16(p0);
-    f.c1 = ld16(p0 + 8);
-    f.c2 = ld16(p0 + 16);
-    f.c3 = ld16(p0 + 24);
-    return f;
+// A lane's 64 bytes of a row's k-block as loaded (two ld_araw), and as operands.
+struct ActRaw {
+    WRaw lo, hi;
+};
+__device__ __forceinline__ ActRaw ld_act(const uint16_t* act, const uint32_t (&off)[2], int kb) {
+    return {ld_araw(act, off, kb * (2 * BLK)), ld_araw(act, off, kb * (2 * BLK) + 32)};
+}
+template <bool PAIR>
+__device__ __forceinline__ Frag16 act_frag(const ActRaw& w) {
+    const v8i l = a_frag<PAIR>(w.lo), h = a_frag<PAIR>(w.hi);
+    return {(v4i){l.s0, l.s1, l.s2, l.s3}, (v4i){l.s4, l.s5, l.s6, l.s7}, (v4i){h.s0, h.s1, h.s2, h.s3},
+            (v4i){h.s4, h.s5, h.s6, h.s7}};
 }
 
 // One 128-deep k-block of a 16 x 16 tile: a . b (+ al . b with PREC, the
@@ -99,14 +103,6 @@ __global__ __launch_bounds__(64 * NW * KS) void gemm2_stream_kernel(
     uint32_t b_off[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) b_off[q] = (uint32_t)((size_t)(n0 + q * 16) * I + wl_off(lane, I));
-    const uint16_t* a_row[MT];
-    const uint16_t* al_row[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        const size_t off = (size_t)(row0 + min(i * 16 + r, nrows - 1)) * I;
-        a_row[i] = p.act + off;
-        al_row[i] = PREC ? p.act_lo + off : nullptr;
-    }
     const float* sb_ptr = w2s + ((size_t)e * HB + nb) * IB;
 
     v4f acc[MT][NQ];
@@ -125,18 +121,26 @@ __global__ __launch_bounds__(64 * NW * KS) void gemm2_stream_kernel(
     // VGPRs for the 64-column waves; 156 with the markers).
     auto body = [&](auto nt) __attribute__((always_inline)) {
         constexpr bool NT = decltype(nt)::value;
+        constexpr bool PAIR = !NT;  // an expert with more than this row tile
         asm volatile("; weight load policy %0 begin" ::"n"(NT ? 1 : 0));
         WRaw b[D][NQ];
-        Frag16 a[D][MT];
-        Frag16 al[D][MT];  // PREC only
+        ActRaw a[D][MT];
+        ActRaw al[D][MT];  // PREC only
+        uint32_t a_off[MT][2];  // (byte offsets of act rows fit 32 bits)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            a_offs<PAIR>(lane, (uint32_t)(row0 + min(i * 16 + r, nrows - 1)) * (2 * I), 64, a_off[i]);
 
         auto compute = [&](int d, int kb) __attribute__((always_inline)) {
             const float sb = sb_ptr[kb_first + kb];
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
+                const Frag16 fa = act_frag<PAIR>(a[d][i]);
+                Frag16 fl;
+                if constexpr (PREC) fl = act_frag<PAIR>(al[d][i]);
 #pragma unroll
                 for (int q = 0; q < NQ; ++q) {
-                    const v4f pr = mfma_block<PREC>(a[d][i], al[d][i], wl_frag(b[d][q]));
+                    const v4f pr = mfma_block<PREC>(fa, fl, wl_frag(b[d][q]));
                     acc[i][q][0] += pr[0] * sb;
                     acc[i][q][1] += pr[1] * sb;
                     acc[i][q][2] += pr[2] * sb;
@@ -146,11 +150,11 @@ __global__ __launch_bounds__(64 * NW * KS) void gemm2_stream_kernel(
         };
         auto load = [&](int d, int kb) __attribute__((always_inline)) {
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) b[d][q] = ld_wraw<NT>(wr, b_off[q] + (kb_first + kb) * BLK, 8 * I);
+            for (int q = 0; q < NQ; ++q) b[d][q] = ld_wraw<NT>(wr, b_off[q] + (kb_first + kb) * BLK, I);
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
-                a[d][i] = ld_act(a_row[i], kb_first + kb, g);
-                if constexpr (PREC) al[d][i] = ld_act(al_row[i], kb_first + kb, g);
+                a[d][i] = ld_act(p.act, a_off[i], kb_first + kb);
+                if constexpr (PREC) al[d][i] = ld_act(p.act_lo, a_off[i], kb_first + kb);
             }
         };
 

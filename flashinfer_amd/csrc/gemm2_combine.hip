@@ -105,7 +105,7 @@ __global__ __launch_bounds__(256) void gemm2_combine_kernel(Plan p, const uint8_
             if (s % KBW == 0 && s > 0) fetch_unit(u0 + ustep * (s / KBW));
             // whole-line weight loads (wl_frag), activation at the same k offsets
             const __amdgpu_buffer_rsrc_t wr = wrsrc(w2 + (size_t)lu.e * H * I, (uint32_t)((size_t)H * I));
-            b[d] = ld_wraw<NT>(wr, (uint32_t)((size_t)n0 * I + wl_off(lane, I) + kb * BLK), 8 * I);
+            b[d] = ld_wraw<NT>(wr, (uint32_t)((size_t)n0 * I + wl_off(lane, I) + kb * BLK), I);
             const size_t ao = (size_t)(lu.row0 + min(r, lu.nrows - 1)) * I + kb * BLK + g * 32;
             const uint16_t* ap = p.act + ao;
             a[d][0] = ld16(ap);

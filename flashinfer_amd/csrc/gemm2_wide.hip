@@ -96,7 +96,7 @@ __global__ __launch_bounds__(64 * W2_NW) void gemm2_wide_kernel(Plan p, const ui
     for (int m = 0; m < MTW; ++m) acc[m] = zero;
 
     auto load_w = [&](int d, int kb) __attribute__((always_inline)) {
-        b[d] = ld_wraw<false>(wr, b_off + kb * BLK, 8 * I);
+        b[d] = ld_wraw<false>(wr, b_off + kb * BLK, I);
     };
     auto load_a = [&](int s, int kb) __attribute__((always_inline)) {
 #pragma unroll

@@ -287,6 +287,7 @@ __device__ __forceinline__ int table_tiles(const WaveTable& w) {
 // t) that picked e.
 struct WaveTile {
     int e, row0, nrows, rank0;
+    int count;  // rows of expert e over all its tiles
     unsigned long long hits;
 };
 
@@ -300,6 +301,7 @@ __device__ __forceinline__ WaveTile table_tile(const WaveTable& w, int lane, int
     t.rank0 = (mt - t0) * bm;
     t.row0 = __builtin_amdgcn_readlane(w.s0, ee) + t.rank0;
     t.nrows = min(bm, ce - t.rank0);
+    t.count = ce;
     t.hits = __ballot((w.m >> ee) & 1);
     return t;
 }

@@ -461,6 +461,24 @@ def test_wide_variants_large(name, variant, monkeypatch):
     _check_output(wl, out, spread_tokens(wl.T, 48))
 
 
+# Decode batches whose experts hold more than one 16-row tile: plain weight loads
+# and activation rows by lane pairs, the last tile with 1 to 16 rows.
+@pytest.mark.parametrize("T", [17, 18, 31, 32, 33, 47, 48, 49, 63, 64])
+@pytest.mark.parametrize("shape", [(7168, 2048), (4096, 1536)])
+def test_decode_several_row_tiles(shape, T, monkeypatch):
+    """Every token on the same 8 experts: the default call has the bits of the
+    separate sort launch, whose GEMM1 keeps one load policy and loads each lane's
+    own row, and the oracle's values."""
+    log(f"test_decode_several_row_tiles[{shape}:{T}]")
+    wl = W.make_workload(f"same_{T}", T=T, seed=7000 + T, skew=True, H=shape[0], I=shape[1])
+    monkeypatch.delenv("MI_MOE_VARIANT", raising=False)
+    out = run_gpu(wl, fill=float("nan")).clone()
+    _check_output(wl, out, spread_tokens(T, 6))
+    monkeypatch.setenv("MI_MOE_SORT_IN_GEMM1", "0")
+    split = run_gpu(wl, fill=float("nan"))
+    assert torch.equal(out.view(torch.int16), split.view(torch.int16))
+
+
 # Rows per expert around what GEMM1's tile does differently: 64 rows a wave group
 # in tiles of at most 128 rows, then 4 or 8 row tiles in the second group, then
 # a second row tile of either form.
