@@ -279,21 +279,25 @@ constexpr int64_t kStreamMaxSlotsPerExpert = 8;
 Variants pick_variants(int64_t T) {
     Variants v;
     // Measured on MI355X: streaming workgroups (GEMM1 with K split over 4
-    // waves) while an expert has at most a few row tiles, 64-column GEMM2 waves from T = 64, the
+    // waves) while an expert has at most a few row tiles, the
     // wide kernels (register-ring weights, LDS activations) for roughly 5 to
     // 70 rows per expert (GEMM2 from ~10 to ~15), the LDS-tiled kernels beyond.
     // GEMM2 with the combine (K split over its 4 waves, which keeps them all
     // busy with fewer than 4 row tiles): one launch fewer where launches
     // dominate (T <= 4). From T = 1 on the K-split GEMM1 (per call with two
     // local slots: 27.9 against 35.6 us for single-wave workgroups, 0.4 us
-    // slower with none); at 7168 x 2048 the K-split 32-column GEMM2 waves up
-    // to T = 16: with random routing T = 12 30.8 against 37.0 us for 64-column
-    // waves, T = 16 77.1 against 79.3; with every token on the same 8 experts
-    // (16 activation rows per tile, which 32-column waves re-read twice as
-    // often) T = 16 83.9 against 77.0, T = 32 158.6 against 139.0.
+    // slower with none). GEMM2 below T = 64: 32-column waves with K split over
+    // 4, which keep 4 times the waves of 64-column ones in flight (per call,
+    // alternating, random routing: T = 18 75.4 against 77.9 us, T = 32 96.9
+    // against 100.9, T = 48 108.7 / 114.5, T = 63 109.9 / 114.8; at H = 4096,
+    // I = 1536 T = 12 31.6 / 33.3, T = 60 55.7 / 56.6, with 16 of 128 experts
+    // T = 12 25.7 / 28.7, T = 60 25.7 / 28.8). With every token on the same 8
+    // experts they lose 3-5 % (T = 32 108.9 against 105.0), since they read the
+    // activation rows twice as often; at T = 64 the two are level with random
+    // routing, and from there on the 64-column waves stay.
     if (T <= 4) v = {16, VARIANT_GEMM2_COMBINE_KS};
     else if (T <= 8 && kSmallLayer) v = {16, 5};
-    else if (T <= 16 && !kSmallLayer) v = {16, 16};
+    else if (T < 64) v = {16, 16};
     else if (T <= 64) v = {16, 14};
     else if (kSmallLayer && T * TOPK <= kStreamMaxSlotsPerExpert * EG) v = {16, 14};
     else if (T <= 128) v = {15, 14};  // the wide GEMM1 folds in the sort from T = 65
