@@ -712,7 +712,7 @@ def main():
         "value": head["us_per_call"], "unit": "us/call", "n_gpus": 1, "steps": a.steps,
         "warmup": a.warmup, "ms_per_step": round(head["us_per_call"] / 1000.0, 5),
         "higher_is_better": False, "scaling": "weak", "vs_baseline": None,
-        "dtype": "fp8_e4m3 (GEMM1) / bf16, or pairs of fp8_e4m3 at full prefill tiles (GEMM2), fp32 accumulate",
+        "dtype": "fp8_e4m3 (GEMM1) / bf16 (GEMM2), fp32 accumulate",
         "data": "synthetic (seeded N(0,1) fp8 weights/activations, U scales, N(0,0.1) bias)",
         "config": {"workload": f"{wl.name}: one fused-MoE layer call, T={wl.T} tokens", "T": wl.T,
                    "H": H, "I": I, "experts_global": E_GLOBAL, "experts_local": 32, "top_k": 8,

@@ -45,13 +45,6 @@ constexpr int64_t kMaxTokens = MI_MOE_MAX_TOKENS;
 static_assert((uint64_t)kMaxTokens * H <= (1ull << 32), "GEMM1 tile row offsets fit 32 bits");
 static_assert((uint64_t)kMaxTokens * TOPK * I * 2 <= (1ull << 32), "GEMM2 tile row offsets fit 32 bits");
 
-// Whether the sort may choose e4m3 pairs for act (pairs_pay) at T tokens: from
-// about 128 slots per expert on, and only where both GEMMs default to LDS tiles
-// (below, GEMM1 may be the wide kernel, which writes bf16). With fewer slots
-// the choice falls on bf16 nearly always, and the second GEMM2 launch, which
-// then finds no tiles, costs ~2 us of a call of ~200.
-constexpr bool act_pair_sized(int64_t T) { return T > 1536 && T * TOPK >= (int64_t)128 * EG; }
-
 constexpr size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Largest T whose GEMM2 writes fp32 partial rows: the workspace reserves
@@ -69,11 +62,6 @@ constexpr int64_t F32_PART_MAX_T = MI_MOE_F32_PART_MAX_T;
 constexpr int64_t SPLIT_ACT_MAX_T = 256;
 static_assert(SPLIT_ACT_MAX_T <= F32_PART_MAX_T, "the split activation writes fp32 rows");
 
-// Bytes of the e4m3 pairs' exponents (Plan::act_sc), which lie before act.
-constexpr size_t act_sc_bytes(int64_t T) {
-    return act_pair_sized(T) ? align_up((size_t)TOPK * (size_t)T * IB * 4) : 0;
-}
-
 constexpr mi_moe_layout make_layout(int64_t T) {
     mi_moe_layout L{};
     const size_t t = (size_t)(T < 0 ? 0 : T);
@@ -88,7 +76,6 @@ constexpr mi_moe_layout make_layout(int64_t T) {
     L.chunk_cnt = o;  o = align_up(o + (size_t)sort_chunks((int)t) * EL * 4);
     const bool f32 = (int64_t)t <= F32_PART_MAX_T;
     const bool split = (int64_t)t <= SPLIT_ACT_MAX_T;
-    o += act_sc_bytes(T);
     L.act = o;        o = align_up(o + s_max * I * 2);
     L.part = o;       o = align_up(o + s_max * H * (f32 ? 4 : 2));
     L.act_lo = o;     o = align_up(o + (split ? s_max * I * 2 : 0));
@@ -170,7 +157,6 @@ Plan make_plan(void* workspace, const mi_moe_layout& L, int64_t T, int64_t local
     p.part = (uint16_t*)(ws + L.part);
     p.part_f32 = nullptr;
     p.act_lo = nullptr;
-    p.act_sc = nullptr;
     p.g1_alt_bm = 0;
     p.g1_mtile = META_MTILE1;
     return p;
@@ -349,8 +335,6 @@ Variants pick_variants(int64_t T) {
     if (env_flag("MI_MOE_G1_SELECT") == 0) v.g1_alt = -1;
     return v;
 }
-
-bool act_pairs(int64_t T, const Variants& v) { return act_pair_sized(T) && v.g1 == 19 && v.g2 == 21; }
 
 }  // namespace
 
@@ -531,7 +515,6 @@ static int run_impl(const mi_moe_args* a, hipStream_t s, hipEvent_t const* ev,
     const int g2_mode = gemm2_mode_for(T, var.g2);
     if (g2_mode != G2_BF16) p.part_f32 = (float*)p.part;
     if (g2_mode == G2_SPLIT) p.act_lo = (uint16_t*)((uint8_t*)a->workspace + L.act_lo);
-    if (act_pairs(T, var)) p.act_sc = (uint32_t*)((uint8_t*)p.act - act_sc_bytes(T));
     hipError_t err = hipSuccess;
     // mark(i) opens phase i (0 route, 1 sort, 2 GEMM1, 3 GEMM2, 4 combine)
     // and closes phase i - 1; the named ranges join route and sort.
@@ -609,9 +592,6 @@ static int run_impl(const mi_moe_args* a, hipStream_t s, hipEvent_t const* ev,
             err = launch_gemm2(p, a->gemm2_weights, a->gemm2_weights_scale,
                                (var.g2 == VARIANT_GEMM2_COMBINE ||
                                 var.g2 == VARIANT_GEMM2_COMBINE_KS) ? 0 : var.g2, s);
-        // the kernel of the other act format, on its own row-tile table
-        if (err == hipSuccess && p.act_sc)
-            err = launch_gemm2_pair(p, a->gemm2_weights, a->gemm2_weights_scale, s);
     }
     mark(4);
     if (err == hipSuccess && !fused) err = launch_combine(p, (uint16_t*)a->output, s);

@@ -100,14 +100,6 @@ struct Plan {
     // act + act_lo, 16 mantissa bits (the reference's fp32 -> TF32 operand
     // keeps 10, kernel.py:272-278).
     uint16_t* act_lo;          // bf16 [TOPK*T, I] or null
-    // act_sc, when set: the sort decides from the expert counts (META_G2_PAIR)
-    // whether act holds bf16 or each SwiGLU value x as two e4m3 numbers, hi +
-    // lo / 16, times a power of two that 32 columns share: per slot and
-    // 128-column block 128 bytes of hi, then 128 of lo, and in act_sc the four
-    // E8M0 exponents of its 32-column blocks. hi keeps x to 4 bits, lo the
-    // remainder to 4 more: at most 2^-9 of x off (bf16: 2^-8), down to 2^-14 of
-    // the block's largest value.
-    uint32_t* act_sc;          // [I / 128][TOPK*T] or null
     // GEMM1 kernel chosen on the device from the expert counts (0: off). When
     // set, the sort also writes the row-tile prefix for tiles of g1_alt_bm rows
     // (META_MTILE1B) and zeroes the total of the table it does not choose, so
@@ -130,9 +122,7 @@ constexpr int META_MTILE1 = META_STRIDE;
 constexpr int META_MTILE2 = 2 * META_STRIDE;
 constexpr int META_MTILE1B = 3 * META_STRIDE;  // GEMM1 row tiles of g1_alt_bm rows
 constexpr int META_G1_SEL = 4 * META_STRIDE;   // 1: the alternative GEMM1 tile was chosen
-constexpr int META_G2_PAIR = META_G1_SEL + 1;  // 1: act handed over as e4m3 pairs
-constexpr int META_MTILE2B = 4 * META_STRIDE + 64;  // GEMM2 row tiles of GEMM2_PAIR_BM rows
-constexpr int META_INTS = 5 * META_STRIDE + 64;
+constexpr int META_INTS = 4 * META_STRIDE + 64;
 
 // Device-side GEMM1 choice (Plan::g1_alt_bm): the LDS tile of g1_alt_bm rows
 // runs instead of the 64-row wide kernel when the 64-row tiling would stream
@@ -142,16 +132,6 @@ constexpr int META_INTS = 5 * META_STRIDE + 64;
 // passes): thresholds of 11 and 12 came within 23.6 us in total of the
 // better kernel on every batch, against 218 us for the wide kernel alone.
 constexpr int G1_SELECT_EXTRA_TILES = 11;
-
-// Device-side choice of the act format (Plan::act_sc set): pairs and the
-// 256-row GEMM2 tile where the slots fill at least 2/3 of the rows of its
-// tiles, bf16 and the 128-row tile where experts are smaller. GEMM2 alone,
-// pairs against bf16 (one process, medians): 99 % full (T=14000 with every
-// token on 8 experts) 2,703 against 3,126 us; 73 % (T=6000) 384 against 403;
-// 70 % (T=8192) 373 against 399; 53 % (T=4096) 264 against 251; 24 % (T=2048)
-// 128 against 126.
-constexpr int GEMM2_PAIR_BM = 256;
-__device__ __forceinline__ bool pairs_pay(int slots, int tiles) { return 3 * slots >= 2 * GEMM2_PAIR_BM * tiles; }
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
@@ -179,14 +159,6 @@ __device__ __forceinline__ v4f mfma_f8_16x16x128(v8i a, v8i b, v4f c) {
 
 __device__ __forceinline__ v4f mfma_bf16_16x16x32(v8bf a, v8bf b, v4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// The same with E8M0 scales: byte SEL of sa scales every block of a; lane l's
-// sb scales the 32-k block l / 16 (bytes [32 (l / 16), +32) of a row's 128)
-// of row l % 16 of b.
-template <int SEL>
-__device__ __forceinline__ v4f mfma_mx_16x16x128(v8i a, int sa, v8i b, int sb, v4f c) {
-    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, SEL, sa, 0, sb);
 }
 
 // Two fp8 e4m3 values (low or high 16 bits of w) -> two bf16, exact.
@@ -477,9 +449,6 @@ hipError_t launch_gemm2_tile(const Plan& p, const uint8_t* w2, const float* w2s,
                              hipStream_t s);
 hipError_t launch_gemm1_wide(const Plan& p, const uint8_t* hs, const float* hs_scale,
                              const uint8_t* w1, const float* w1s, hipStream_t s);
-// GEMM2 from act as e4m3 pairs (Plan::act_sc), bf16 partial rows, on the
-// row-tile table META_MTILE2B (empty where the device kept bf16).
-hipError_t launch_gemm2_pair(const Plan& p, const uint8_t* w2, const float* w2s, hipStream_t s);
 hipError_t launch_gemm2_wide(const Plan& p, const uint8_t* w2, const float* w2s, hipStream_t s);
 
 // GEMM kernel variants: 0/1/2 weight-streaming with 16/32/64-row tiles and

@@ -451,76 +451,17 @@ struct G1P {
     static_assert(HB <= 64 && HB >= 2, "weight scales: one lane per k-block");
 };
 
-// Values a, b as e4m3 (round to nearest even), in the low 16 bits.
-__device__ __forceinline__ uint32_t pk_e4m3(float a, float b) {
-    return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false) & 0xffffu;
+// End of a phase: this wave's LDS reads are done and at most N of its copies
+// are outstanding; then the workgroup's barrier.
+template <int N>
+__device__ __forceinline__ void phase_end() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void phase_end() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// Eight SwiGLU values of one row into the e4m3 pairs of Plan::act_sc: x[n][v]
-// is column 16n + 4g + v of the 32-column block that lanes r, r + 16, r + 32
-// and r + 48 of the wave hold together. d: the hi and lo dwords of n = 0, then
-// of n = 1; returns the block's exponent byte. hi is the value at a scale that
-// puts the block's largest in [128, 256), lo 16 times what hi leaves (at most
-// 128, exact in fp32). A block with an infinity keeps it infinite (448 x 2^127
-// overflows in the product) and drops its finite values; a NaN stays NaN.
-__device__ __forceinline__ uint32_t split_e4m3(const float (&x)[2][4], uint32_t (&d)[4]) {
-    uint32_t am = 0;
-#pragma unroll
-    for (int n = 0; n < 2; ++n)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) am = max(am, __builtin_bit_cast(uint32_t, x[n][v]) & 0x7fffffffu);
-    {
-        const auto a = __builtin_amdgcn_permlane32_swap(am, am, false, false);
-        am = max(a[0], a[1]);
-        const auto b = __builtin_amdgcn_permlane16_swap(am, am, false, false);
-        am = max(b[0], b[1]);
-    }
-    const uint32_t ex = min(max(am >> 23, 8u), 254u);
-    const float up = __builtin_bit_cast(float, (261u - ex) << 23);  // 2^(7 - exponent)
-    float y[2][4];
-#pragma unroll
-    for (int n = 0; n < 2; ++n)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) y[n][v] = x[n][v] * up;
-    uint32_t sc = ex - 7u;
-    if (am >= 0x7f800000u) {
-        sc = 254u;
-#pragma unroll
-        for (int n = 0; n < 2; ++n)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float f = x[n][v];
-                y[n][v] = f != f ? f : (__builtin_isinf(f) ? __builtin_copysignf(448.f, f) : 0.f);
-            }
-    }
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-        const uint32_t h = pk_e4m3(y[n][0], y[n][1]) | (pk_e4m3(y[n][2], y[n][3]) << 16);
-        d[2 * n] = h;
-        const float r0 = (y[n][0] - __builtin_amdgcn_cvt_f32_fp8(h, 0)) * 16.f;
-        const float r1 = (y[n][1] - __builtin_amdgcn_cvt_f32_fp8(h, 1)) * 16.f;
-        const float r2 = (y[n][2] - __builtin_amdgcn_cvt_f32_fp8(h, 2)) * 16.f;
-        const float r3 = (y[n][3] - __builtin_amdgcn_cvt_f32_fp8(h, 3)) * 16.f;
-        d[2 * n + 1] = pk_e4m3(r0, r1) | (pk_e4m3(r2, r3) << 16);
-    }
-    return sc;
-}
-
-// 4 x 4 transpose over the lanes r, r + 16, r + 32, r + 48: lane group g gets
-// in d[j] what group j held in d[g].
-__device__ __forceinline__ void transpose4(uint32_t (&d)[4]) {
-    const auto a = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
-    const auto b = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
-    const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
-    const auto e = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
-    d[0] = c[0];
-    d[1] = c[1];
-    d[2] = e[0];
-    d[3] = e[1];
-}
-
-// PAIR: act may be e4m3 pairs instead of bf16 (Plan::act_sc).
-template <int GM, bool PAIR>
+template <int GM>
 __global__ __launch_bounds__(512) void gemm1_tile_p_kernel(
     Plan p, const uint8_t* __restrict__ hs, const float* __restrict__ hs_scale,
     const uint8_t* __restrict__ w1, const float* __restrict__ w1s) {
@@ -541,7 +482,6 @@ __global__ __launch_bounds__(512) void gemm1_tile_p_kernel(
     const int r = lane & 15, g = lane >> 4;
     const int jb = nt * C::BG;
     const bool small = nrows <= 128;
-    const bool pair = PAIR && p.meta[META_G2_PAIR] != 0;
 
     auto token = [&](int row) __attribute__((always_inline)) {
         return (uint32_t)p.sorted_tok[row0 + min(row, nrows - 1)];
@@ -566,8 +506,13 @@ __global__ __launch_bounds__(512) void gemm1_tile_p_kernel(
         if (lane < HB) g2l4s(w1s + ((size_t)e * N1B + nb) * HB, lane * 4, s_sb + (wave - 4) * 64);
     }
 
-    const FragOff fo(r, g);
-    auto frag = [&](const uint8_t* s) __attribute__((always_inline)) { return lds_frag(s, fo); };
+    // fragment of 16 rows at s: this lane's row r, 16-byte chunks g and g + 4
+    const int lo_off = r * BLK + ((g ^ swzq(r)) << 4), hi_off = r * BLK + (((g + 4) ^ swzq(r)) << 4);
+    auto frag = [&](const uint8_t* s) __attribute__((always_inline)) {
+        const v4i lo = lds16(s + lo_off);
+        const v4i hi = lds16(s + hi_off);
+        return (v8i){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    };
     // weight rows of column tile n (0, 1 gate; 2, 3 up) in a stage's weight region
     auto bcol = [&](int n) __attribute__((always_inline)) {
         return (n < 2 ? 32 * wn + 16 * n : C::BG + 32 * wn + 16 * (n - 2)) * BLK;
@@ -609,40 +554,21 @@ __global__ __launch_bounds__(512) void gemm1_tile_p_kernel(
             asm volatile("" : "+v"(acc[m][0]), "+v"(acc[m][1]), "+v"(acc[m][2]), "+v"(acc[m][3]));
     };
     auto store_row = [&](int row, const v4f (&a)[4]) __attribute__((always_inline)) {
-        if (PAIR && pair) {
-            // the four lanes of a row exchange their pieces, so that each
-            // stores 16 bytes: hi, lo of columns 0-15, hi, lo of 16-31
-            float x[2][4];
+        if (row >= nrows) return;
 #pragma unroll
-            for (int n = 0; n < 2; ++n)
+        for (int n = 0; n < 2; ++n) {
+            uint32_t w[2], wl[2];
 #pragma unroll
-                for (int v = 0; v < 4; ++v) x[n][v] = silu(a[n + 2][v]) * a[n][v];
-            uint32_t d[4];
-            const uint32_t sc = split_e4m3(x, d);
-            transpose4(d);
-            if (row >= nrows) return;
-            uint8_t* o = reinterpret_cast<uint8_t*>(p.act) + (size_t)(row0 + row) * (2 * I) + nt * (2 * BLK) +
-                         (g & 1) * BLK + wn * 32 + (g >> 1) * 16;
-            *reinterpret_cast<uint4*>(o) = make_uint4(d[0], d[1], d[2], d[3]);
-            if (g == 0)
-                reinterpret_cast<uint8_t*>(p.act_sc + (size_t)nt * ((size_t)TOPK * p.T) + row0 + row)[wn] = (uint8_t)sc;
-        } else {
-            if (row >= nrows) return;
-#pragma unroll
-            for (int n = 0; n < 2; ++n) {
-                uint32_t w[2], wl[2];
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const float v0 = silu(a[n + 2][2 * h]) * a[n][2 * h];
-                    const float v1 = silu(a[n + 2][2 * h + 1]) * a[n][2 * h + 1];
-                    const uint16_t h0 = f2bf(v0), h1 = f2bf(v1);
-                    w[h] = (uint32_t)h0 | ((uint32_t)h1 << 16);
-                    wl[h] = (uint32_t)f2bf(v0 - bf2f(h0)) | ((uint32_t)f2bf(v1 - bf2f(h1)) << 16);
-                }
-                const size_t idx = (size_t)(row0 + row) * I + jb + wn * 32 + n * 16 + 4 * g;
-                *reinterpret_cast<uint2*>(p.act + idx) = make_uint2(w[0], w[1]);
-                if (p.act_lo) *reinterpret_cast<uint2*>(p.act_lo + idx) = make_uint2(wl[0], wl[1]);
+            for (int h = 0; h < 2; ++h) {
+                const float v0 = silu(a[n + 2][2 * h]) * a[n][2 * h];
+                const float v1 = silu(a[n + 2][2 * h + 1]) * a[n][2 * h + 1];
+                const uint16_t h0 = f2bf(v0), h1 = f2bf(v1);
+                w[h] = (uint32_t)h0 | ((uint32_t)h1 << 16);
+                wl[h] = (uint32_t)f2bf(v0 - bf2f(h0)) | ((uint32_t)f2bf(v1 - bf2f(h1)) << 16);
             }
+            const size_t idx = (size_t)(row0 + row) * I + jb + wn * 32 + n * 16 + 4 * g;
+            *reinterpret_cast<uint2*>(p.act + idx) = make_uint2(w[0], w[1]);
+            if (p.act_lo) *reinterpret_cast<uint2*>(p.act_lo + idx) = make_uint2(wl[0], wl[1]);
         }
     };
 
@@ -858,13 +784,8 @@ hipError_t launch_gemm1_tile(const Plan& p, const uint8_t* hs, const float* hs_s
         // a time and copy 1.5x the distinct lines of 4 x 8 (T=14000 with every
         // token on 8 experts 2,755 against 2,705 us; T=8192 level).
         const int tiles = max_mtiles(p.T, G1P::BM) * G1P::NT;
-        const dim3 grid((tiles + 7) / 8 * 8);
-        if (p.act_sc)
-            hipLaunchKernelGGL((gemm1_tile_p_kernel<8, true>), grid, dim3(G1P::THREADS), 0, s, p, hs,
-                               hs_scale, w1, w1s);
-        else
-            hipLaunchKernelGGL((gemm1_tile_p_kernel<8, false>), grid, dim3(G1P::THREADS), 0, s, p, hs,
-                               hs_scale, w1, w1s);
+        hipLaunchKernelGGL((gemm1_tile_p_kernel<8>), dim3((tiles + 7) / 8 * 8), dim3(G1P::THREADS), 0,
+                           s, p, hs, hs_scale, w1, w1s);
     } else if (variant == 18) {
         using C = G1Tile<4, 2>;
         const int tiles = max_mtiles(p.T, C::BM) * C::NT;

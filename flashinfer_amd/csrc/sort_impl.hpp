@@ -55,7 +55,7 @@ __device__ __forceinline__ TokLocal load_local(const int* ids_base, const float*
 // expert offsets and the row-tile prefixes for GEMM tiles of bm1 / bm2 rows.
 __device__ __forceinline__ int scan_counts(const Plan& p, int lane, int c, int bm1, int bm2,
                                            bool write) {
-    const int bm3 = p.g1_alt_bm > 0 ? p.g1_alt_bm : p.act_sc ? GEMM2_PAIR_BM : bm1;
+    const int bm3 = p.g1_alt_bm > 0 ? p.g1_alt_bm : bm1;
     int v0 = c, v1 = (c + bm1 - 1) / bm1, v2 = (c + bm2 - 1) / bm2, v3 = (c + bm3 - 1) / bm3;
     const int own0 = v0, own1 = v1, own2 = v2, own3 = v3;
 #pragma unroll
@@ -73,23 +73,14 @@ __device__ __forceinline__ int scan_counts(const Plan& p, int lane, int c, int b
         const int t1 = __shfl(v1, EL - 1);
         alt = t1 - active >= G1_SELECT_EXTRA_TILES ? 1 : 0;
     }
-    // Device-side choice of the act format and with it of the GEMM2 kernel
-    // (uniform; never together with the GEMM1 choice).
-    const bool pair_choice = p.act_sc != nullptr && p.g1_alt_bm == 0;
     if (write && lane < EL) {
         p.meta[META_EXPERT_OFF + lane] = v0 - own0;
         p.meta[META_MTILE1 + lane] = v1 - own1;
         p.meta[META_MTILE2 + lane] = v2 - own2;
         if (p.g1_alt_bm > 0) p.meta[META_MTILE1B + lane] = v3 - own3;
-        if (pair_choice) p.meta[META_MTILE2B + lane] = v3 - own3;
         if (lane == EL - 1) {
             p.meta[META_EXPERT_OFF + EL] = v0;
-            const bool pair = pair_choice && pairs_pay(v0, v3);
-            p.meta[META_MTILE2 + EL] = pair ? 0 : v2;
-            if (pair_choice) {
-                p.meta[META_MTILE2B + EL] = pair ? v3 : 0;
-                p.meta[META_G2_PAIR] = pair ? 1 : 0;
-            }
+            p.meta[META_MTILE2 + EL] = v2;
             // the table of the kernel not chosen holds no tiles
             p.meta[META_MTILE1 + EL] = alt ? 0 : v1;
             if (p.g1_alt_bm > 0) {

@@ -52,26 +52,6 @@ __device__ __forceinline__ void g2l4s(const void* sbase, uint32_t voff, void* ld
                  : "memory", "m0");
 }
 
-// 16-byte buffer -> LDS copy through a buffer resource (soffset counts in its
-// range check): an offset past the resource's end writes zeros and reads no
-// memory.
-__device__ __forceinline__ void b2l16(v4i rsrc, uint32_t voff, uint32_t soff, void* lds_base) {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 :
-                 : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_addr(lds_base))
-                 : "memory", "m0");
-}
-
-// End of a phase of the two-group tiles: this wave's LDS reads are done and at
-// most N of its copies are outstanding; then the workgroup's barrier.
-template <int N>
-__device__ __forceinline__ void phase_end() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void phase_end() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 __device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // XOR swizzle of the 16-byte chunk index inside a 128-byte LDS row: 16
@@ -87,25 +67,10 @@ __device__ __forceinline__ int swz8(int row) { return (row & 7) ^ ((row >> 3) & 
 // x 8 chunks still reads each row's 128 bytes whole.
 __device__ __forceinline__ int swzq(int row) { return (((row >> 2) & 3) << 1) | ((row >> 1) & 1); }
 
-// Byte offset of lane (r = lane % 16, g = lane / 16)'s two 16-byte chunks g
-// and g + 4 of row r in a 128-byte-row LDS region with swzq rows.
-struct FragOff {
-    int lo, hi;
-    __device__ __forceinline__ FragOff(int r, int g)
-        : lo(r * BLK + ((g ^ swzq(r)) << 4)), hi(r * BLK + (((g + 4) ^ swzq(r)) << 4)) {}
-};
-
 // Same for a 256-byte row of 16 chunks.
 __device__ __forceinline__ int swz16(int row) { return row & 15; }
 
 __device__ __forceinline__ v4i lds16(const uint8_t* p) { return *reinterpret_cast<const v4i*>(p); }
-
-// The fp8 MFMA operand of 16 such rows starting at s.
-__device__ __forceinline__ v8i lds_frag(const uint8_t* s, FragOff o) {
-    const v4i lo = lds16(s + o.lo);
-    const v4i hi = lds16(s + o.hi);
-    return (v8i){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-}
 
 // Logical tile order shared by the tiled GEMMs. Tiles of one expert are
 // visited in groups of GM row tiles; inside a group every n tile is swept

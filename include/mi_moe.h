@@ -84,12 +84,7 @@ typedef struct mi_moe_args {
  *   sorted_w   fp32  [kT]     routing weight of each slot
  *   tok_slot   int32 [T, 8]   slots of each token, ascending local expert, -1 pad
  *   chunk_cnt  int32 [ceil(T/256), E]   per-256-token-chunk local expert counts
- *   act        bf16  [kT, 2048]  SwiGLU(GEMM1) per slot, rounded to bf16; from
- *                             about 128 slots per expert on, where the counts
- *                             fill 256-row tiles, the same bytes hold it as two
- *                             e4m3 numbers (per 128 columns 128 bytes of hi, 128 of
- *                             lo; value (hi + lo / 16) x 2^e), whose exponents
- *                             e, one per 32 columns, lie before act
+ *   act        bf16  [kT, 2048]  SwiGLU(GEMM1) per slot, rounded to bf16
  *   part       bf16  [kT, 7168]  routing weight x GEMM2 row per slot; fp32
  *                             (same offset, twice the bytes) at T <= 1024
  *   act_lo     bf16  [kT, 2048]  SwiGLU(GEMM1) - act, reserved at T <= 256

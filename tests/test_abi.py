@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from flashinfer_amd import _lib, kernel
+from flashinfer_amd.shapes import DEFINITIONS
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -69,6 +70,21 @@ def test_workspace_layout_monotone_and_aligned():
         assert L.total == _lib.workspace_size(T) and L.total > prev
         assert L.total - L.part >= 8 * T * 7168 * 2
         prev = L.total
+
+
+@pytest.mark.parametrize("defn", DEFINITIONS, ids=lambda d: d.name)
+def test_workspace_holds_the_documented_regions_only(defn):
+    """The regions lie one after the other at the header's sizes, each rounded
+    up to 256 bytes, up to act: no region without a field of its own."""
+    up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    for T in (1, 64, 1025, 1537, 2731, 2816, 4095, 4096, 8192, 14000, 65536):
+        L = _lib.workspace_layout(T, defn)
+        slots = defn.TOPK * T
+        assert L.topk_w - L.topk_ids == L.expert_off - L.topk_w == up(T * 32), T
+        assert L.sorted_w - L.sorted_tok == L.tok_slot - L.sorted_w == up(slots * 4), T
+        assert L.chunk_cnt - L.tok_slot == up(T * 32), T
+        assert L.act - L.chunk_cnt == up(-(-T // 256) * defn.EL * 4), T
+        assert L.part - L.act == up(slots * defn.I * 2), T
 
 
 def test_workspace_reserves_fp32_rows_to_1024_and_act_lo_to_256():
