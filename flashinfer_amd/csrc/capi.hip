@@ -262,6 +262,18 @@ Front pick_front(int64_t T, int g1) {
 constexpr bool kSmallLayer = (int64_t)H * I < (int64_t)7168 * 2048;
 constexpr int64_t kStreamMaxSlotsPerExpert = 8;
 
+// Slots (T * top_k) up to which the K-split GEMM2's waves take 32 columns
+// rather than 64. Twice the waves are ahead while an expert has few row tiles;
+// beyond, 32-column waves read every activation row twice as often, which tells
+// when the tokens share experts. Per call, 32 against 64 columns: at 7168 x
+// 2048 random routing T = 17 78.2 against 79.3 us, T = 32 98.7 / 99.5, T = 48
+// 112.4 / 113.8, T = 63 113.7 / 115.0, but on the same 8 experts T = 17 98.1 /
+// 95.5, T = 32 109.1 / 104.2, T = 48 139.2 / 130.7, T = 63 170.6 / 159.3. At
+// H = 4096, I = 1536, random / same: T = 32 60.2 against 61.7 / 45.3 against
+// 43.9, T = 40 60.8, 61.7 / 57.3, 54.7, T = 63 62.7, 63.3 / 72.9, 68.5; with 16
+// of 128 experts T = 40 26.3, 27.1 / 45.7, 44.8, T = 48 26.0, 27.0 / 52.9, 51.5.
+constexpr int64_t kNarrowMaxSlots = kSmallLayer ? 256 : 128;
+
 Variants pick_variants(int64_t T) {
     Variants v;
     // Measured on MI355X: streaming workgroups (GEMM1 with K split over 4
@@ -272,18 +284,20 @@ Variants pick_variants(int64_t T) {
     // busy with fewer than 4 row tiles): one launch fewer where launches
     // dominate (T <= 4). From T = 1 on the K-split GEMM1 (per call with two
     // local slots: 27.9 against 35.6 us for single-wave workgroups, 0.4 us
-    // slower with none). GEMM2 below T = 64: 32-column waves with K split over
-    // 4, which keep 4 times the waves of 64-column ones in flight (per call,
-    // alternating, random routing: T = 18 75.4 against 77.9 us, T = 32 96.9
-    // against 100.9, T = 48 108.7 / 114.5, T = 63 109.9 / 114.8; at H = 4096,
-    // I = 1536 T = 12 31.6 / 33.3, T = 60 55.7 / 56.6, with 16 of 128 experts
-    // T = 12 25.7 / 28.7, T = 60 25.7 / 28.8). With every token on the same 8
-    // experts they lose 3-5 % (T = 32 108.9 against 105.0), since they read the
-    // activation rows twice as often; at T = 64 the two are level with random
-    // routing, and from there on the 64-column waves stay.
+    // slower with none). GEMM2 below T = 64: K split over 4 waves, which keeps 4
+    // times the waves of whole-K ones in flight; 32 columns a wave up to
+    // kNarrowMaxSlots slots, 64 columns above (kNarrowMaxSlots says why).
+    // Per call against 64-column waves with whole K (variant 14), alternating,
+    // at 7168 x 2048, random routing: T = 17 79.3 against 80.6 us, T = 32 99.5 /
+    // 100.4, T = 63 115.0 / 115.6, 140.5 / 146.3 and 86.5 / 84.8 on three draws;
+    // every token on the same 8 experts: T = 32 104.2 / 104.9, T = 48 130.7 /
+    // 132.4, T = 63 159.3 / 162.6. At T = 64 the two are within 2 % (115.2 / 115.8; 159.6 /
+    // 163.1 on the same experts), so the line to variant 14 there costs at most
+    // that.
     if (T <= 4) v = {16, VARIANT_GEMM2_COMBINE_KS};
     else if (T <= 8 && kSmallLayer) v = {16, 5};
-    else if (T < 64) v = {16, 16};
+    else if (T * TOPK <= kNarrowMaxSlots) v = {16, 16};
+    else if (T < 64) v = {16, 9};
     else if (T <= 64) v = {16, 14};
     else if (kSmallLayer && T * TOPK <= kStreamMaxSlotsPerExpert * EG) v = {16, 14};
     else if (T <= 128) v = {15, 14};  // the wide GEMM1 folds in the sort from T = 65

@@ -8,10 +8,13 @@ Bars (written in each test):
   oracle's fp32 accumulator, no element outside;
 * determinism: two calls are bit-identical.
 """
+import re
+
 import pytest
 import torch
 
 from flashinfer_amd import workloads as W
+from flashinfer_amd.shapes import DEFINITIONS
 
 from _helpers import log, oracle_subset, run_gpu, spread_tokens, gpu_args
 
@@ -516,6 +519,38 @@ def test_default_variants_by_T(name, T, variant, monkeypatch):
     monkeypatch.setenv("MI_MOE_VARIANT", variant)
     forced = run_gpu(wl, fill=float("nan"))
     assert torch.equal(out.view(torch.int16), forced.view(torch.int16))
+
+
+# The edges of the decode GEMM2's rule: slots at most 128 (256 in smaller layers,
+# where top-6 of 128 reaches them at T = 42), then to T = 63.
+@pytest.mark.parametrize("defn,T,columns", [
+    (DEFINITIONS[0], 16, 32), (DEFINITIONS[0], 17, 64), (DEFINITIONS[0], 63, 64),
+    (DEFINITIONS[1], 32, 32), (DEFINITIONS[1], 33, 64), (DEFINITIONS[1], 63, 64),
+    (DEFINITIONS[3], 42, 32), (DEFINITIONS[3], 43, 64)],
+    ids=lambda x: x.name if hasattr(x, "name") else str(x))
+def test_decode_gemm2_waves(defn, T, columns, monkeypatch):
+    """GEMM2 splits K over four waves of 32 columns up to the rule's slots and of
+    64 above: 32-column waves read each activation row twice as often, which
+    costs 3-5 % when tokens share experts. The default call runs that kernel
+    and gives the bits of the variant forced, and the oracle's values."""
+    from flashinfer_amd import kernel
+    log(f"test_decode_gemm2_waves[{defn.name}:{T}]")
+    wl = W.make_for(defn, f"waves_{T}", T, 8000 + T)
+    wl.tensors["routing_logits"][:, :defn.TOPK] += 12.0  # every token on the same experts
+    wl.tensors["routing_bias"].zero_()
+    monkeypatch.delenv("MI_MOE_VARIANT", raising=False)
+    out = run_gpu(wl, fill=float("nan")).clone()
+    args, again = gpu_args(wl), torch.empty_like(out)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        kernel.run(*args, again)
+        torch.cuda.synchronize()
+    forms = [m for e in prof.key_averages()
+             for m in re.findall(r"gemm2_stream_kernel<(\d+), (\d+), (\d+), (\d+), (\d+), (\d+)>", e.key)]
+    assert [(16 * int(f[3]), int(f[5])) for f in forms] == [(columns, 4)], forms
+    monkeypatch.setenv("MI_MOE_VARIANT", "16,16" if columns == 32 else "16,9")
+    forced = run_gpu(wl, fill=float("nan"))
+    assert torch.equal(out.view(torch.int16), forced.view(torch.int16))
+    _check_output(wl, out, spread_tokens(T, 6))
 
 
 @pytest.mark.parametrize("name,T,extra", [("c2_t1024_o0", 1024, {}), ("c2_t1024_o64", 1024, {}),
