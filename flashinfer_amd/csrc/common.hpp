@@ -208,11 +208,11 @@ __device__ __forceinline__ v4i ld16(const void* p) { return *reinterpret_cast<co
 // The pair matters: the address unit takes a contiguous run of lanes per
 // clock, so neighbouring lanes in different rows move 16 bytes a clock and CU
 // whatever cache answers (9.7 TB/s over the card from L2; 19 TB/s by pairs, 30
-// by fours, which would take 2.5 times the exchange). Weights and activations
-// together ran into that in every streaming kernel: T=64 GEMM1 moved 0.88 GB
-// through it, 91 us at 9.7 TB/s. Per call, one process each, weights by pairs
-// against lanes 8 rows apart: T=1 28.7 against 31.7 us, T=4 47.1 / 50.9, T=16
-// 61.0 / 64.8, T=64 87.5 / 93.0.
+// by fours, which would take 2.5 times the exchange). Per call, alternating
+// processes, weights by pairs against lanes 8 rows apart, three draws of random
+// routing each: T=1 28.8 against 31.8 us, 22.7 / 24.8, 31.0 / 34.9; T=4 47.2 /
+// 51.0, 24.3 / 26.4, 24.0 / 25.8; T=16 98.5 / 102.1, 61.3 / 64.8, 52.5 / 54.9;
+// T=64, where HBM is the nearer bound, 111.2 / 114.5, 112.3 / 115.3, 87.5 / 93.3.
 __device__ __forceinline__ size_t wl_off(int lane, size_t row_stride) {
     return (size_t)(lane & 14) * row_stride + (lane >> 4) * 32 + (lane & 1) * 16;
 }
@@ -235,8 +235,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t wrsrc(const void* base, uint32
 // argument: per workgroup from its expert's row count in the wide GEMM1, the
 // stream GEMM2 and the stream GEMM1's front forms (two copies of the k loop,
 // BoolC below; T=64 with every token on 8 experts, four 16-row tiles each:
-// GEMM1 102 against 135 us with the hint); per launch from T (wt_nt) in the
-// other stream GEMM1 forms and in the GEMM2 + combine kernel.
+// GEMM1 102 against 135 us with the hint); per launch from T in the other
+// stream GEMM1 forms (wt_nt) and in the GEMM2 + combine kernel (no second
+// 16-row tile: T <= 16). The wide GEMM2 loads plainly.
 struct WRaw {
     v4i x, y;
 };
@@ -249,14 +250,15 @@ __device__ __forceinline__ WRaw ld_wraw(__amdgpu_buffer_rsrc_t r, uint32_t off, 
     return w;
 }
 
-// Weight load policy of a launch with T tokens and `bm`-row tiles: non-
+// Weight load policy of a stream GEMM1 launch with T tokens and `bm`-row tiles
+// (its front forms then still load plainly where an expert has several): non-
 // temporal while an expert holds about one row tile or less on average
 // (T * top_k <= bm * global experts / 4: T <= 128 for 16-row tiles, 512 for
 // 64-row tiles with the default routing; a shard's experts can hold twice
 // the uniform share, as at T = 1024 offset 0). Measured per GEMM with random
-// routing at T = 16 / 64 / 100 / 256 / 512: 9-12 % faster with the hint;
-// with every token on the same 8 experts (T = 64 / 256: 4 row tiles each)
-// 5-7 % slower, the price of not knowing the counts on the host.
+// routing at T = 16 / 64 / 100 / 256 / 512: 9-12 % faster with the hint.
+// Where the counts come from a sort launch, the host does not know them: with
+// every token on the same 8 experts the hint then costs the re-reads from HBM.
 inline bool wt_nt(int64_t T, int bm) { return T * TOPK <= (int64_t)bm * EG / 4; }
 
 // Compile-time bool for `body(BoolC<NT>{})`: a kernel whose register budget

@@ -412,8 +412,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm1_tile_t_kernel(
 // time): 2,657 cycles a k-block now against about 4,450 before, 2,048 of
 // them MFMA. The rest is power: with random data the clock falls to 1.6-1.8
 // GHz in this loop (2.1-2.2 in the same loop without its copies), so bytes
-// and operations saved count as much as cycles. GEMM1 alone, one process: T=14000 with every
-// token on 8 experts 3,010 -> 2,695 us, T=8192 458 -> 420 us (medians).
+// and operations saved count as much as cycles. GEMM1 by events, alternating
+// processes: T=14000 with every token on 8 experts 2,925 -> 2,585 us, T=8192
+// 416 -> 372, T=2048 192 -> 185, T=1024 with 1,966 slots 202 -> 194.
 //
 // Copies (two stages): the weights and row tiles 0-3 of k-block kb + 2 go out
 // in M1 of kb, after both groups have read theirs of kb (group 1 in the slot
@@ -424,9 +425,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm1_tile_t_kernel(
 // of C0 / C1, for group 1, one slot behind, the end of M0 / M1.
 //
 // A tile of at most 128 rows gives each group 64 of them (M, C; two phases a
-// k-block, a third of the activation copies) and uses the LDS for three
-// stages. An expert's last row tile is often one: at T=1000 (19 row tiles)
-// 144 -> 133 us.
+// k-block, half the activation copies) and uses the LDS for three stages. An
+// expert's last row tile is often one.
 //
 // MFMA operands are swapped as in variant 18 (weights are the A operand, so a
 // lane holds four output columns of one row and one scale factor per tile),
