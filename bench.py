@@ -18,10 +18,11 @@ call captured in a HIP graph, and the probes of libmi_peaks.so measure the
 HBM and MFMA rates this GPU achieves.
 
 Rank 0 prints ONE JSON line. ``roofline`` covers the dominant kernel
-(GEMM1+SwiGLU; at T=8192 bound by FP8 MFMA), with HBM traffic and the MFMA
-busy fraction from rocprofv3 counter passes; ``kernels`` gives both GEMMs'
-rooflines; ``call_roofline`` the whole call; ``sweep`` every configuration
-(the headline included), each with its dominant kernel's roofline, a
+(the GEMM launch that takes longest; at T=8192 both are bound by MFMA), with
+its HBM traffic and MFMA busy fraction from rocprofv3 counter passes;
+``kernels`` gives both GEMMs' rooflines; ``call_roofline`` the whole call;
+``sweep`` every configuration (the headline included), each with its
+dominant kernel's roofline, a
 ``parity`` block and, at the CPU reference configuration (T=16) and the
 metric's points (T = 1 with and without a local slot, 256, 8192), the CPU
 oracle timed on this host (``cpu_baseline``); ``quantize_fp8`` the
@@ -519,10 +520,16 @@ def _pick(per_kernel, key):
     return statistics.median(xs) if xs else None
 
 
-def pmc_counters(workload, kernel_key, copy_mib=1024, timeout=240):
-    """Counters of the first kernel whose name contains ``kernel_key``, from
-    three rocprofv3 passes over short child runs of this bench (each pass a
-    process of its own): HBM bytes per launch from FETCH_SIZE and WRITE_SIZE,
+def counter_keys(T):
+    """What the names of the two GEMM kernels contain at T tokens (GEMM1,
+    GEMM2): LDS tiles above T = 1536, streaming or wide kernels below."""
+    return ("gemm1_tile", "gemm2_tile") if T > 1536 else ("gemm1_", "gemm2_")
+
+
+def pmc_counters(workload, *kernel_keys, copy_mib=1024, timeout=240):
+    """Per key of ``kernel_keys``, counters of the kernels whose name contains
+    it, from three rocprofv3 passes over short child runs of this bench (each
+    pass a process of its own): HBM bytes per launch from FETCH_SIZE and WRITE_SIZE,
     each scaled to bytes by what the same counter reads for a device copy of
     ``copy_mib`` MiB timed in the same pass; and the MFMA busy fraction,
     SQ_VALU_MFMA_BUSY_CYCLES per SIMD (1024 SIMDs) over GRBM_GUI_ACTIVE per
@@ -534,30 +541,42 @@ def pmc_counters(workload, kernel_key, copy_mib=1024, timeout=240):
         return None
     if shutil.which("rocprofv3") is None:
         return None
-    out = {"kernel_key": kernel_key, "copy_bytes": copy_mib << 20}
-    for counter in ("FETCH_SIZE", "WRITE_SIZE"):
-        vals = _pmc_pass([counter], workload, copy_mib, timeout)
-        key = "fetch" if counter == "FETCH_SIZE" else "write"
-        k_units = _pick(vals[counter], kernel_key) if vals else None
-        c_units = max((v for name, vs in vals[counter].items() if "copyBuffer" in name
-                       for v in vs), default=None) if vals else None
-        if k_units is None or not c_units:
-            out[f"{key}_bytes"] = None
-            continue
-        scale = (copy_mib << 20) / c_units
-        out[f"{key}_counter"] = k_units
-        out[f"{key}_copy_counter"] = c_units
-        out[f"{key}_scale"] = round(scale, 4)
-        out[f"{key}_bytes"] = k_units * scale
-    fb, wb = out.get("fetch_bytes"), out.get("write_bytes")
-    out["bytes"] = fb + wb if fb is not None and wb is not None else None
-    vals = _pmc_pass(["SQ_VALU_MFMA_BUSY_CYCLES", "GRBM_GUI_ACTIVE"], workload, 0, timeout)
-    busy = _pick(vals["SQ_VALU_MFMA_BUSY_CYCLES"], kernel_key) if vals else None
-    gui = _pick(vals["GRBM_GUI_ACTIVE"], kernel_key) if vals else None
-    out["mfma_busy_cycles"] = busy
-    out["gui_active_cycles"] = gui
-    out["mfma_busy_frac"] = round((busy / 1024) / (gui / 8), 4) if busy and gui else None
-    return out
+    sizes = {c: _pmc_pass([c], workload, copy_mib, timeout) for c in ("FETCH_SIZE", "WRITE_SIZE")}
+    busy_pass = _pmc_pass(["SQ_VALU_MFMA_BUSY_CYCLES", "GRBM_GUI_ACTIVE"], workload, 0, timeout)
+    res = {}
+    for kernel_key in kernel_keys:
+        out = res[kernel_key] = {"kernel_key": kernel_key, "copy_bytes": copy_mib << 20}
+        for counter, vals in sizes.items():
+            key = "fetch" if counter == "FETCH_SIZE" else "write"
+            k_units = _pick(vals[counter], kernel_key) if vals else None
+            c_units = max((v for name, vs in vals[counter].items() if "copyBuffer" in name
+                           for v in vs), default=None) if vals else None
+            if k_units is None or not c_units:
+                out[f"{key}_bytes"] = None
+                continue
+            scale = (copy_mib << 20) / c_units
+            out[f"{key}_counter"] = k_units
+            out[f"{key}_copy_counter"] = c_units
+            out[f"{key}_scale"] = round(scale, 4)
+            out[f"{key}_bytes"] = k_units * scale
+        fb, wb = out.get("fetch_bytes"), out.get("write_bytes")
+        out["bytes"] = fb + wb if fb is not None and wb is not None else None
+        busy = _pick(busy_pass["SQ_VALU_MFMA_BUSY_CYCLES"], kernel_key) if busy_pass else None
+        gui = _pick(busy_pass["GRBM_GUI_ACTIVE"], kernel_key) if busy_pass else None
+        out["mfma_busy_cycles"] = busy
+        out["gui_active_cycles"] = gui
+        out["mfma_busy_frac"] = round((busy / 1024) / (gui / 8), 4) if busy and gui else None
+    return res
+
+
+def with_counters(roof, counters, T):
+    """A roofline entry with the HBM traffic and MFMA busy fraction of its own
+    kernel (``counters`` of pmc_counters, or None)."""
+    if not counters:
+        return dict(roof, traffic=None)
+    c = counters[counter_keys(T)[0 if roof["kernel"] == "gemm1_swiglu" else 1]]
+    return dict(roof, traffic=round(c["bytes"]) if c.get("bytes") else None,
+                mfma_busy_frac=c.get("mfma_busy_frac"))
 
 
 def host_cores():
@@ -621,12 +640,9 @@ def main():
         sys.exit(2)
     counters = None
     if not a.no_pmc and not a.vendor_gemm_ref:
-        # counter passes run as child processes before this one uses the GPU;
-        # the dominant kernel at the headline is the LDS-tiled GEMM1 above
-        # T = 1536, the K-split or wide GEMM1 below
+        # counter passes run as child processes before this one uses the GPU
         from flashinfer_amd import workloads as W
-        key = "gemm1_tile" if W.STANDARD[a.workload]["T"] > 1536 else "gemm1_"
-        counters = pmc_counters(a.workload, key)
+        counters = pmc_counters(a.workload, *counter_keys(W.STANDARD[a.workload]["T"]))
     if not torch.cuda.is_available():
         print("bench.py needs a ROCm GPU", file=sys.stderr)
         sys.exit(2)
@@ -694,12 +710,7 @@ def main():
     for r in sweep:
         r.pop("_check", None)
 
-    roof = dict(head["roofline"])
-    if counters:
-        roof["traffic"] = round(counters["bytes"]) if counters.get("bytes") else None
-        roof["mfma_busy_frac"] = counters.get("mfma_busy_frac")
-    else:
-        roof["traffic"] = None
+    roof = with_counters(head["roofline"], counters, wl.T)
     if peaks and roof.get("bound") == "mfma":
         meas = peaks["fp8_mfma_tflops"] if roof.get("mfma_dtype") == "fp8" else peaks["bf16_mfma_tflops"]
         roof["measured_peak"] = meas

@@ -53,6 +53,24 @@ def test_counter_passes_never_start_under_a_profiler(monkeypatch):
     assert not bench.profiler_inherited({})
 
 
+def test_counters_belong_to_the_kernel_of_the_roofline(monkeypatch):
+    """The passes count both GEMMs; the printed traffic and MFMA busy fraction
+    are those of the kernel the roofline names, whichever GEMM takes longest."""
+    g1, g2, copy = "mimoe::gemm1_tile_p_kernel<8>", "mimoe::gemm2_tile_w_kernel<4, 0, true>", "copyBuffer"
+    passes = {"FETCH_SIZE": {g1: [30.0, 31.0, 30.0], g2: [20.0], copy: [2.0 ** 20]},
+              "WRITE_SIZE": {g1: [2.0], g2: [4.0], copy: [2.0 ** 21]},
+              "SQ_VALU_MFMA_BUSY_CYCLES": {g1: [1024.0], g2: [1024.0]},
+              "GRBM_GUI_ACTIVE": {g1: [16.0], g2: [32.0]}}
+    monkeypatch.setattr(bench, "_pmc_pass", lambda c, *a: {k: passes[k] for k in c})
+    monkeypatch.setattr(bench, "profiler_inherited", lambda: False)
+    monkeypatch.setattr(bench.shutil, "which", lambda name: "/opt/rocm/bin/" + name)
+    counters = bench.pmc_counters("c3_t8192", *bench.counter_keys(8192))
+    for kernel, traffic, busy in (("gemm1_swiglu", 30 * 1024 + 2 * 512, 0.5), ("gemm2", 20 * 1024 + 4 * 512, 0.25)):
+        roof = bench.with_counters({"kernel": kernel, "frac": 0.5}, counters, 8192)
+        assert roof == {"kernel": kernel, "frac": 0.5, "traffic": traffic, "mfma_busy_frac": busy}
+    assert bench.with_counters({"kernel": "gemm2"}, None, 8192) == {"kernel": "gemm2", "traffic": None}
+
+
 def test_parity_block_pass_and_planted_error():
     """The parity fields the bench prints per workload: the oracle's own bf16
     output passes with zero routing mismatches; a planted error in one
